@@ -51,6 +51,7 @@ struct WriteArgs {
     uint32_t log2_cpr, log2_il, log2_pcp, log2_block;  // when POW2
     uint32_t num_tokens;
     uint32_t first_pos;
+    uint32_t next_chunk;  // positions from the last one of a rank's chunk to its next chunk's first (at most 2^31)
     int32_t max_local_blocks;
     int32_t num_pages;
     int32_t head_dim;
@@ -128,7 +129,23 @@ __global__ void __launch_bounds__(kThreads) kv_write_kernel(WriteArgs a, uint32_
     const int32_t entry = (int32_t)(owner * a.max_local_blocks + blk);
     const int32_t page = table_page(a.block_table, entry, a.table_shift);
     if ((uint32_t)page >= (uint32_t)a.num_pages) return;
-    if (a.page_valid_len && head == 0 && chunk == 0) atomicMax(a.page_valid_len + entry, (int32_t)slot + 1);
+    if (a.page_valid_len && head == 0 && chunk == 0) {
+        // Only the entry's last token of the range raises its length (a
+        // rank's slots grow with the position): the last slot of the block,
+        // or a token whose rank's next position lies past the range.  One
+        // atomic per token queued up to block_size of them on one address:
+        // the full 64-rank e4m3 history (131072 tokens) took 188 us with
+        // them and takes 66 us without, 1000 tokens 13.9 and 3.4 us.
+        const uint32_t p = p0 + token;
+        uint32_t in_chunk;
+        if constexpr (POW2)
+            in_chunk = p & ((1u << a.log2_il) - 1);
+        else
+            in_chunk = local - div(local, a.interleave) * a.interleave.d;
+        const uint32_t next = in_chunk + 1 == a.interleave.d ? p + a.next_chunk : p + 1;
+        if (slot + 1 == a.block.d || next - p0 >= a.num_tokens)
+            atomicMax(a.page_valid_len + entry, (int32_t)slot + 1);
+    }
 
     const int64_t src = ((int64_t)row * a.head_dim + chunk * 8) * 2;  // [Hkv, n, D] bf16
     const v4i kin = *(const v4i*)(a.k + src);

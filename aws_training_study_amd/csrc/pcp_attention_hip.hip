@@ -632,6 +632,8 @@ int32_t pcpa_kv_cache_write(const pcpa_params* p, int32_t interleave, int64_t fi
     a.log2_block = pow2 ? l_blk : 0;
     a.num_tokens = (uint32_t)num_tokens;
     a.first_pos = (uint32_t)first_pos;
+    const int64_t next_chunk = (int64_t)(p->pcp_size - 1) * interleave + 1;
+    a.next_chunk = (uint32_t)(next_chunk < (1ll << 31) ? next_chunk : (1ll << 31));
     a.max_local_blocks = p->max_local_blocks;
     a.num_pages = p->num_pages;
     a.head_dim = p->head_dim;
