@@ -455,6 +455,16 @@ __device__ __forceinline__ void tile_step(const FwdArgs& a, const TileCursor& cu
 // the guard plan, -1 past its fix_count rows), whether it exists, its rank
 // and local token, and the byte offset of its Q and output rows in [pcp, Hq,
 // local_q, D] bf16.
+// CAUSAL: rows are taken in the order (round of chunks, rank, Q head of the
+// group, token of the chunk) instead of (rank, Q head, token), i.e. by
+// global position up to one chunk.  A workgroup's rows then share a chunk or
+// two, so that its walk ends where all of them end, and later row tiles
+// never have less work than earlier ones, which the heaviest-first launch
+// order relies on whatever the striping (one round, local_q = interleave, is
+// the same order either way).  In (rank, Q head, token) order a tile of 16
+// ranks x 256 local tokens mixed chunks 1024 positions apart and its limit
+// followed the tile's parity, not its index: 4096 current tokens at head_dim
+// 256 took 504 us, now 357.
 struct QueryRow {
     int row;
     bool ok;
@@ -462,7 +472,7 @@ struct QueryRow {
     int tok;
     int64_t off;
 };
-template <int D, bool FIXUP>
+template <int D, bool FIXUP, bool CAUSAL = false>
 __device__ __forceinline__ QueryRow query_row(const FwdArgs& a, int head, int row_tile, int pw, int j, int fix_first,
                                               int fix_count) {
     QueryRow r;
@@ -475,10 +485,22 @@ __device__ __forceinline__ QueryRow query_row(const FwdArgs& a, int head, int ro
         r.row = row_tile * kRowsPerGroup + pw * kRowsPerWave + j;
     r.ok = FIXUP ? r.row >= 0 : r.row < a.rows_per_head;
     const int rowc = r.ok ? r.row : (FIXUP ? 0 : a.rows_per_head - 1);
-    r.rank = rowc / a.group_rows;
-    const int rem = rowc - r.rank * a.group_rows;
-    const int head_in_group = rem / a.local_q;
-    r.tok = rem - head_in_group * a.local_q;
+    int head_in_group;
+    if constexpr (CAUSAL) {
+        const int chunk_rows = a.group * a.interleave;  // rows of one chunk of one rank
+        const int chunk = rowc / chunk_rows;            // in global order
+        int rem = rowc - chunk * chunk_rows;
+        const int round = chunk / a.pcp;
+        r.rank = chunk - round * a.pcp;
+        head_in_group = rem / a.interleave;
+        rem -= head_in_group * a.interleave;
+        r.tok = round * a.interleave + rem;
+    } else {
+        r.rank = rowc / a.group_rows;
+        const int rem = rowc - r.rank * a.group_rows;
+        head_in_group = rem / a.local_q;
+        r.tok = rem - head_in_group * a.local_q;
+    }
     r.off = ((int64_t)(r.rank * a.num_q_heads + head * a.group + head_in_group) * a.local_q + r.tok) * D * 2;
     return r;
 }
@@ -584,7 +606,7 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
     const int gl = lane & 15;
 
     // ---- this lane's query row -------------------------------------------
-    const QueryRow qr = query_row<D, FIXUP>(a, head, row_tile, pw, j, fix_first, fix_count);
+    const QueryRow qr = query_row<D, FIXUP, CAUSAL>(a, head, row_tile, pw, j, fix_first, fix_count);
     const int rank = qr.rank, tok = qr.tok;
     const uint8_t* const qrow = a.q + qr.off;
 
