@@ -312,14 +312,20 @@ __device__ __forceinline__ void dma_vaddr(const uint8_t* addr, uint32_t m0v) {
                  : "memory", "m0");
 }
 
-// Four bf16 values (8 bytes) widened exactly from four e4m3 codes (one dword).
-__device__ __forceinline__ v2i e4m3x4_to_bf16x4(int codes) {
-    const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(codes, false);
-    const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(codes, true);
-    // e4m3 values are exact in bf16: keep the upper half of each f32.
-    const int w0 = (int)((__float_as_uint(lo[0]) >> 16) | (__float_as_uint(lo[1]) & 0xffff0000u));
-    const int w1 = (int)((__float_as_uint(hi[0]) >> 16) | (__float_as_uint(hi[1]) & 0xffff0000u));
-    return v2i{w0, w1};
+// D = A B + C of 32x32x64 with e4m3 operands, and of 32x32x16 with bf16 ones.
+__device__ __forceinline__ v16f mfma_e4m3(const v8i& a, const v8i& b, const v16f& c) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+}
+__device__ __forceinline__ v16f mfma_bf16(const v4i& a, const v8bf& b, const v16f& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), b, c, 0, 0, 0);
+}
+
+// Eight bf16 values widened from eight e4m3 codes (exact; a scale of 1).
+__device__ __forceinline__ v4i e4m3x8_to_bf16x8(int lo, int hi) {
+    return v4i{__builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, false)),
+               __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, true)),
+               __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, false)),
+               __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, true))};
 }
 
 // s_waitcnt vmcnt(0) with expcnt/lgkmcnt left unconstrained (gfx9 encoding).
@@ -356,6 +362,27 @@ __device__ __forceinline__ v2i ds_read_tr16_b64(uint32_t addr) {
     v2i r;
     asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
     return r;
+}
+template <int OFF>
+__device__ __forceinline__ v4i ds_read_b128(uint32_t addr) {
+    static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
+    v4i r;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
+    return r;
+}
+// s_waitcnt lgkmcnt(N) with the awaited read results as operands, so that
+// no use of them is scheduled before the wait.
+template <int N>
+__device__ __forceinline__ void lds_wait(v4i& x) {
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "i"(N));
+}
+template <int N>
+__device__ __forceinline__ void lds_wait(v4i (&x)[2]) {
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(x[0]), "+v"(x[1]) : "i"(N));
+}
+template <int N>
+__device__ __forceinline__ void lds_wait(v2i (&x)[4]) {
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]) : "i"(N));
 }
 // s_waitcnt lgkmcnt(0), with the read results as operands so that no use of
 // them (and no copy of the registers) can be scheduled before the wait.

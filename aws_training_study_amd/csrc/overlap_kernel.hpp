@@ -20,23 +20,6 @@ constexpr float kMaxFloor = -1.0e30f;
 // partial tile that lie past its valid length.
 __device__ __attribute__((aligned(16))) uint8_t zero_chunk[16];
 
-template <int OFF>
-__device__ __forceinline__ v4i ds_read_b128(uint32_t addr) {
-    static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
-    v4i r;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
-    return r;
-}
-// s_waitcnt lgkmcnt(N) with the awaited read results as operands, so that
-// no use of them is scheduled before the wait.
-template <int N>
-__device__ __forceinline__ void lds_wait(v4i (&x)[2]) {
-    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(x[0]), "+v"(x[1]) : "i"(N));
-}
-template <int N>
-__device__ __forceinline__ void lds_wait(v2i (&x)[4]) {
-    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]) : "i"(N));
-}
 // max(a, b, c) in one v_max3_f32, without the NaN-quieting moves the
 // compiler adds around fmaxf of accumulator reads.  Inputs are scores or
 // -inf, never NaN.
@@ -384,7 +367,7 @@ __device__ __forceinline__ void s_half(uint32_t k_addr, uint32_t v_addr, const v
         }
         const v4i lo = kr[op & 1][0], hi = kr[op & 1][1];
         const v8i kop = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        s[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kop, q[c], c == 0 ? v16f{} : s[t], 0, 0, 0, 0, 0, 0);
+        s[t] = mfma_e4m3(kop, q[c], c == 0 ? v16f{} : s[t]);
         if constexpr (op == 1) {
             // The row sum has long completed (two score MFMAs since): read
             // it, then free its registers.  All 4 stay allocated until the
@@ -427,7 +410,7 @@ __device__ __forceinline__ void pv_half(uint32_t v_addr, v2i (&xv0)[4], v16f (&o
         lds_wait<0>(x);
         if constexpr (dt + 1 < S::DT) issue_v(std::integral_constant<int, dt + 1>{});
         const v8i vop = {x[0][0], x[0][1], x[1][0], x[1][1], x[2][0], x[2][1], x[3][0], x[3][1]};
-        o[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vop, p_old, o[dt], 0, 0, 0, 0, 0, 0);
+        o[dt] = mfma_e4m3(vop, p_old, o[dt]);
         after_mfma(dc);
         softmax_slices<S::pv_begin(dt), S::pv_begin(dt + 1), FAST>(s, p_new, sm);
         __builtin_amdgcn_sched_barrier(0);

@@ -7,53 +7,59 @@
 namespace pcpa {
 
 // STORE8: the cache holds e4m3 (else bf16).  FP8: the MFMAs run on e4m3
-// operands (requires STORE8); otherwise they run on bf16, and an e4m3 cache
-// is widened to bf16 while it is staged into LDS.
+// operands (requires STORE8); otherwise on bf16 ones.  An e4m3 cache with bf16
+// MFMAs (WIDE) keeps its tiles in e4m3 in LDS, with the e4m3 paths' layout and
+// operand maps, and widens each operand exactly between its LDS read and its
+// MFMAs: K and V then cost half the LDS reads and DMA of a bf16 cache, and the
+// conversions (one per two elements) issue under the wave's own MFMAs.
+// Widening while staging instead, through registers, could not use the
+// LDS-DMA, nor overlap the next tile's loads: 16 ranks x 1024 tokens over 8192
+// keys at head_dim 256 took 309 us a call that way and take 229 (64% of the
+// bf16 MFMA peak at the clock held; the softmax finds few MFMAs of the other
+// wave on its SIMD to run under).  Two e4m3 terms for Q and P instead of
+// widened K and V are as fast but sum less exactly: the e4m3 MFMA's products
+// are not added in full fp32 (log-sum-exp off by 1.6e-4 where bf16 MFMAs give
+// under 1e-4).
 template <int D, bool STORE8, bool FP8>
 struct TileShape {
     static_assert(STORE8 || !FP8, "e4m3 MFMAs need an e4m3 cache");
-    static constexpr int ES = FP8 ? 1 : 2;
-    static constexpr bool F8 = FP8;
-    static constexpr int ROW = D * ES;                 // LDS bytes of one key row
+    static constexpr bool MFMA8 = FP8;
+    static constexpr bool F8 = STORE8;                 // e4m3 tile layout and operand maps
+    static constexpr bool WIDE = STORE8 && !FP8;       // e4m3 tiles, bf16 MFMAs
+    static constexpr int ES = F8 ? 1 : 2;
+    static constexpr int ROW = D * ES;                 // LDS and cache bytes of one key row
     static constexpr int CHUNKS = ROW / 16;
     static constexpr int TILE = kKeyTile * ROW;        // LDS bytes of one K (or V) tile
-    static constexpr int GROW = D * (STORE8 ? 1 : 2);  // cache bytes of one key row
-    static constexpr int GCHUNKS = GROW / 16;
-    static constexpr bool WIDEN = STORE8 && !FP8;
-    // Double-buffered (prefetching) when both buffers fit in 128 KB of LDS
-    // (gfx950 has 160 KB per CU); the widening path stages synchronously
-    // through registers.
-    static constexpr int NBUF = (!WIDEN && 4 * TILE <= 131072) ? 2 : 1;
     static constexpr int QK = FP8 ? D / 64 : D / 16;   // k-steps of the score MFMA
     static constexpr int DT = D / 32;                  // 32-row d tiles of O^T
-    // BF16 MFMAs at head_dim 256 run eight waves in key-split pairs: the two
-    // waves of a SIMD take the same 32 rows and one half of every tile's
-    // keys each, with an online softmax and O^T of their own, merged
-    // through LDS at the end.  (One wave holding all 64 keys of a tile
-    // needs 448 registers, i.e. one wave per SIMD and nothing to overlap
-    // the softmax with.)
+    // BF16 precision at head_dim 256 runs eight waves in pairs: the two waves
+    // of a SIMD take the same 32 rows and half of the keys each, with an
+    // online softmax and O^T of their own, merged through LDS at the end
+    // (O^T and Q alone take 192 registers a wave).  A bf16 cache: each wave
+    // takes one 32-key half of every tile (all 64 keys need 448 registers,
+    // i.e. one wave per SIMD and nothing to overlap the softmax with).  An
+    // e4m3 cache: each wave takes every other tile, two tiles a step.
     static constexpr bool PAIR = D == 256 && !FP8;
+    static constexpr bool PAIR_HALVES = PAIR && !WIDE;
+    static constexpr int TILES = PAIR && WIDE ? 2 : 1;  // tiles per step (and buffer)
     static constexpr int WAVES = PAIR ? 2 * kWaves : kWaves;
     static constexpr int THREADS = 64 * WAVES;
-    static constexpr int NT = PAIR ? 1 : 2;            // 32-key score tiles per wave and tile
+    static constexpr int NT = PAIR_HALVES ? 1 : 2;     // 32-key score tiles per wave and tile
     static constexpr int DMA_PER_WAVE = CHUNKS / WAVES;  // 1 KB DMA blocks per wave per operand
-    // LDS: the tile buffers, which a PAIR workgroup reuses for the partners'
-    // O^T (32 KB per pair) after the walk.
-    static constexpr int LDS_BYTES = (PAIR && NBUF * 2 * TILE < 4 * 32768) ? 4 * 32768 : NBUF * 2 * TILE;
+    // Two buffers (the next step's tiles load during this one's), which a
+    // PAIR workgroup reuses for the partners' O^T (32 KB per pair) after the
+    // walk.
+    static constexpr int BUFFER = TILES * 2 * TILE;
+    static constexpr int LDS_BYTES = (PAIR && 2 * BUFFER < 4 * 32768) ? 4 * 32768 : 2 * BUFFER;
+    static_assert(LDS_BYTES <= 131072, "gfx950 has 160 KB of LDS per CU");
     // Wave w loads DMA blocks WAVES i + w.  Block i's lane chunk sits
-    // dma_key_delta(i) key rows after block 0's, with the same chunk swizzle,
-    // except for 512-byte rows (bf16 D=256) loaded by four waves, whose
-    // blocks are 8 rows apart and whose swizzle (a function of the row mod
-    // 16) changes between blocks: those keep one offset per block
-    // (DMA_SPLIT).  Eight waves put a wave's blocks 16 rows apart.
-    static constexpr bool DMA_SPLIT = ROW == 512 && WAVES == kWaves;
-    static constexpr int K_T1_ROWS = FP8 ? 16 : 32;    // LDS rows from score tile 0 to tile 1
-    static constexpr int dma_key_delta(int i) {
-        // keys between DMA block i's lane chunk and block 0's (rows are WAVES i 1024 / ROW apart)
-        return FP8 ? (ROW == 256 ? 16 * (i & 1) + 8 * (i >> 1) : ROW == 128 ? 8 * i : 0) : i * WAVES * 1024 / ROW;
-    }
+    // dma_key_delta(i) key rows after block 0's, with the same chunk swizzle
+    // (its LDS rows are a multiple of 16 further on).
+    static_assert(DMA_PER_WAVE == 1 || (WAVES * 1024 / ROW) % 16 == 0, "DMA blocks must share the chunk swizzle");
+    static constexpr int K_T1_ROWS = F8 ? 16 : 32;     // LDS rows from score tile 0 to tile 1
+    static constexpr int dma_key_delta(int i) { return lds_row<F8>(i * WAVES * 1024 / ROW); }
     // Lazy rescale: the running max is only raised when a tile's max exceeds
-    // it by more than this (log2 units); FP8 probabilities then stay below
+    // it by more than this (log2 units); e4m3 probabilities then stay below
     // 2^(kPBiasLog2 + 2.5) = 362 < 448.
     static constexpr float RESCALE_LOG2 = FP8 ? 2.5f : 8.0f;
 };
@@ -67,76 +73,32 @@ __host__ __device__ constexpr int tile_threads(int d, bool fp8) {
 template <class S>
 struct LaneMap {
     uint32_t k_addr;                      // score A operand of tile 0 (tile 1: + K_T1_ROWS rows)
-    uint32_t v_addr[S::ES == 1 ? 1 : 2];  // PV A operand base(s)
-    uint32_t dma_off[S::DMA_SPLIT ? S::DMA_PER_WAVE : 1];   // global byte offset of the lane's K DMA chunk
-    uint32_t dma_off_v[S::DMA_SPLIT ? S::DMA_PER_WAVE : 1]; // same for the V tile (its own swizzle)
+    uint32_t v_addr[S::F8 ? 1 : 2];       // PV A operand base(s)
+    uint32_t dma_off;                     // global byte offset of the lane's K DMA chunk
+    uint32_t dma_off_v;                   // same for the V tile (its own swizzle)
     int rsel;  // e4m3 MFMAs: the row-sum selector operand word (e4m3 1.0 bytes or 0)
 };
 
-// Issue asynchronous global->LDS loads of one 64-key K tile and V tile.  The
-// tile is split into 1 KB blocks; each wave loads DMA_PER_WAVE blocks of
-// each, one 16-byte chunk per lane, landing at block + 16 * lane.  The
-// lane's global chunk (dma_off) is chosen so that the swizzled LDS layout
-// comes out.
-template <class S, int BUF>
-__device__ __forceinline__ void stage_tile_async(const FwdArgs& a, const TileCursor& c, uint8_t* lds, int wave,
+// Issue asynchronous global->LDS loads of one 64-key K tile and V tile to
+// `lk` (K, then V).  The tile is split into 1 KB blocks; each wave loads
+// DMA_PER_WAVE blocks of each, one 16-byte chunk per lane, landing at block +
+// 16 * lane.  The lane's global chunk (dma_off) is chosen so that the swizzled
+// LDS layout comes out.
+template <class S>
+__device__ __forceinline__ void stage_tile_async(const FwdArgs& a, const TileCursor& c, uint8_t* lk, int wave,
                                                  const LaneMap<S>& L) {
-    const uint8_t* const kt = a.kv + c.k_off + (int64_t)c.base * S::GROW;
+    const uint8_t* const kt = a.kv + c.k_off + (int64_t)c.base * S::ROW;
     const uint8_t* const vt = kt + (int64_t)a.num_kv_heads * a.head_stride;
-    uint8_t* const lk = lds + BUF * 2 * S::TILE;
+    // (the opaque base keeps each block's address computation next to its
+    // load: all of them ahead of the first load delay the whole burst)
+    uint32_t dst = lds_address(lk) + wave * 1024;
 #pragma unroll
     for (int i = 0; i < S::DMA_PER_WAVE; ++i) {
-        const int block = S::WAVES * i + wave;
-        const uint32_t koff = L.dma_off[S::DMA_SPLIT ? i : 0];
-        const uint32_t voff = L.dma_off_v[S::DMA_SPLIT ? i : 0];
-        const int delta = S::DMA_SPLIT ? 0 : S::dma_key_delta(i) * S::GROW;
-        dma_sbase<0>(kt + delta, koff, lds_address(lk + block * 1024));
-        dma_sbase<0>(vt + delta, voff, lds_address(lk + S::TILE + block * 1024));
-    }
-}
-
-// Synchronous staging through registers into buffer 0, widening e4m3 to
-// bf16 when the MFMAs are bf16.  Rows at or beyond `valid` get zero V.
-template <class S>
-__device__ __forceinline__ void stage_tile_sync(const FwdArgs& a, const TileCursor& c, int valid, uint8_t* lds,
-                                                int tid) {
-    constexpr int LOADS = kKeyTile * S::GROW / (16 * S::THREADS);
-    static_assert((kKeyTile * S::GROW) % (16 * S::THREADS) == 0, "tile must split into 16-byte chunks per thread");
-    const uint8_t* const kpage = a.kv + c.k_off;
-    const uint8_t* const vpage = kpage + (int64_t)a.num_kv_heads * a.head_stride;
-    uint8_t* const lds_k = lds;
-    uint8_t* const lds_v = lds + S::TILE;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int chunk_id = tid + S::THREADS * i;
-        const int key = chunk_id / S::GCHUNKS;
-        const int ch = chunk_id - key * S::GCHUNKS;
-        const int64_t goff = (int64_t)(c.base + key) * S::GROW + ch * 16;
-        const v4i kc = *(const v4i*)(kpage + goff);
-        v4i vc = *(const v4i*)(vpage + goff);
-        if (key >= valid) vc = v4i{0, 0, 0, 0};
-        const int row = lds_row<S::ES == 1>(key);
-        const int sw = chunk_swizzle<S::ES == 1, S::CHUNKS>(row);
-        const int swv = chunk_swizzle_v<S::ES == 1, S::CHUNKS>(row);
-        if constexpr (S::WIDEN) {
-            // 16 e4m3 codes become 32 bytes (LDS chunks 2ch, 2ch+1).
-            const v2i k0 = e4m3x4_to_bf16x4(kc[0]), k1 = e4m3x4_to_bf16x4(kc[1]);
-            const v2i k2 = e4m3x4_to_bf16x4(kc[2]), k3 = e4m3x4_to_bf16x4(kc[3]);
-            const v2i v0 = e4m3x4_to_bf16x4(vc[0]), v1 = e4m3x4_to_bf16x4(vc[1]);
-            const v2i v2 = e4m3x4_to_bf16x4(vc[2]), v3 = e4m3x4_to_bf16x4(vc[3]);
-            // (K and V rows have swizzles of their own)
-            const int lo = row * S::ROW + (((2 * ch) ^ sw) << 4);
-            const int hi = row * S::ROW + (((2 * ch + 1) ^ sw) << 4);
-            const int lov = row * S::ROW + (((2 * ch) ^ swv) << 4);
-            const int hiv = row * S::ROW + (((2 * ch + 1) ^ swv) << 4);
-            *(v4i*)(lds_k + lo) = v4i{k0[0], k0[1], k1[0], k1[1]};
-            *(v4i*)(lds_k + hi) = v4i{k2[0], k2[1], k3[0], k3[1]};
-            *(v4i*)(lds_v + lov) = v4i{v0[0], v0[1], v1[0], v1[1]};
-            *(v4i*)(lds_v + hiv) = v4i{v2[0], v2[1], v3[0], v3[1]};
-        } else {
-            *(v4i*)(lds_k + row * S::ROW + ((ch ^ sw) << 4)) = kc;
-            *(v4i*)(lds_v + row * S::ROW + ((ch ^ swv) << 4)) = vc;
-        }
+        const int delta = S::dma_key_delta(i) * S::ROW;
+        asm volatile("" : "+s"(dst));
+        dma_sbase<0>(kt + delta, L.dma_off, dst + S::WAVES * i * 1024);
+        asm volatile("" : "+s"(dst));
+        dma_sbase<0>(vt + delta, L.dma_off_v, dst + S::TILE + S::WAVES * i * 1024);
     }
 }
 
@@ -146,7 +108,7 @@ template <class S>
 __device__ __forceinline__ void zero_masked_v(uint8_t* lds_v, int valid, int tid) {
     for (int idx = tid; idx < (kKeyTile - valid) * S::CHUNKS; idx += S::THREADS) {
         const int key = valid + idx / S::CHUNKS;
-        *(v4i*)(lds_v + lds_row<S::ES == 1>(key) * S::ROW + (idx % S::CHUNKS) * 16) = v4i{0, 0, 0, 0};
+        *(v4i*)(lds_v + lds_row<S::F8>(key) * S::ROW + (idx % S::CHUNKS) * 16) = v4i{0, 0, 0, 0};
     }
 }
 
@@ -161,31 +123,56 @@ struct SoftmaxState {
 };
 
 template <class S>
-using QOperand = typename std::conditional<S::ES == 1, v8i, v8bf>::type;
+using QOperand = typename std::conditional<S::MFMA8, v8i, v8bf>::type;
 
-// One 64-key tile held in LDS buffer BUF (PAIR: this wave's 32 keys of it;
-// its operand addresses in L include the half): S^T = K Q^T, masked online
+// One 64-key tile held in LDS buffer BUF (PAIR_HALVES: this wave's 32 keys of
+// it; its operand addresses in L include the half): S^T = K Q^T, masked online
 // softmax, O^T += V^T P^T.  `valid`: the valid keys counted from the wave's
 // first key.
 // CAUSAL: `valid` differs per lane (the row's causal limit within the tile,
 // possibly <= 0).
 //
 // rt_off: a byte offset added to both buffers' addresses at run time (PAIR
-// walks alternate buffers with one loop body, BUF 0 and rt_off 0 or
-// 2 * TILE; otherwise 0).
+// walks alternate buffers with one loop body, BUF 0; otherwise 0).
 template <class S, int BUF, bool CAUSAL = false>
 __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off, int valid,
-                                             const QOperand<S> (&qop)[S::QK], float cscale, const LaneMap<S>& L, int h,
-                                             SoftmaxState<S>& st) {
-    constexpr bool FP8 = S::ES == 1;
+                                             const QOperand<S> (&qop)[S::QK], float cscale,
+                                             const LaneMap<S>& L, int h, SoftmaxState<S>& st) {
+    constexpr bool F8 = S::F8, FP8 = S::MFMA8;
     constexpr int ROW = S::ROW, QK = S::QK, DT = S::DT;
-    constexpr int KBASE = BUF * 2 * S::TILE;
+    constexpr int KBASE = BUF * S::BUFFER;
     constexpr int VBASE = KBASE + S::TILE;
     const uint8_t* const lk = lds + KBASE + rt_off;
 
     // ---- S^T = K . Q^T : two 32-key x 32-query tiles --------------------
     v16f s[2];
-    if constexpr (FP8) {
+    if constexpr (S::WIDE) {
+        // MFMA m takes half m & 1 (8 of 16 codes, one k-step of d) of read
+        // m / 2, whose score tile is the read's parity.  Two reads are in
+        // flight; each half is widened under the MFMA before its own.
+        const uint32_t ka = lds_address(lk) + L.k_addr;
+        constexpr int READS = QK;  // two score tiles x D / 32 chunk pairs
+        v4i raw[2], kop[2];
+        auto issue = [&](auto rc) {
+            constexpr int rd = decltype(rc)::value, c = rd >> 1, t = rd & 1;
+            raw[t] = ds_read_b128<t * S::K_T1_ROWS * ROW>(ka ^ ((2 * c) << 4));
+        };
+        auto widen = [&](auto mc) {
+            constexpr int m = decltype(mc)::value, rd = m >> 1, half = m & 1;
+            if constexpr (half == 0) lds_wait<(rd + 1 < READS ? 1 : 0)>(raw[rd & 1]);
+            kop[m & 1] = e4m3x8_to_bf16x8(raw[rd & 1][2 * half], raw[rd & 1][2 * half + 1]);
+            if constexpr (half == 1 && rd + 2 < READS) issue(std::integral_constant<int, rd + 2>{});
+        };
+        issue(std::integral_constant<int, 0>{});
+        issue(std::integral_constant<int, 1>{});
+        widen(std::integral_constant<int, 0>{});
+        static_for<0, 2 * READS>([&](auto mc) {
+            constexpr int m = decltype(mc)::value, c = m >> 2, t = (m >> 1) & 1, half = m & 1;
+            s[t] = mfma_bf16(kop[m & 1], qop[2 * c + half], c + half == 0 ? v16f{} : s[t]);
+            if constexpr (m + 1 < 2 * READS) widen(std::integral_constant<int, m + 1>{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    } else if constexpr (FP8) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             s[t] = v16f{};
@@ -195,7 +182,7 @@ __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off
                 const v4i lo = *(const v4i*)(kt + (L.k_addr ^ ((4 * c) << 4)));
                 const v4i hi = *(const v4i*)(kt + (L.k_addr ^ ((4 * c + 1) << 4)));
                 const v8i aop = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                s[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aop, qop[c], s[t], 0, 0, 0, 0, 0, 0);
+                s[t] = mfma_e4m3(aop, qop[c], s[t]);
             }
         }
     } else {
@@ -236,11 +223,11 @@ __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off
     if (CAUSAL ? __builtin_amdgcn_ballot_w64(valid < KEYS) != 0 : valid < KEYS) {
         // key_of_acc(t, r, h) >= valid, as its lane-independent part against
         // valid less its lane-half part
-        const int lim = valid - key_of_acc<FP8>(0, 0, h);
+        const int lim = valid - key_of_acc<F8>(0, 0, h);
         const float ninf = -INFINITY;
         static_for<0, 16 * S::NT>([&](auto kc) {
             constexpr int t = decltype(kc)::value >> 4, r = decltype(kc)::value & 15;
-            constexpr int k = FP8 ? 16 * t + r : 32 * t + 16 * (r >> 3) + (r & 7);
+            constexpr int k = F8 ? 16 * t + r : 32 * t + 16 * (r >> 3) + (r & 7);
             s[t][r] = mask_key_at_or_past<k>(s[t][r], lim, ninf);
         });
     }
@@ -278,7 +265,45 @@ __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off
 
     __builtin_amdgcn_s_setprio(S::PAIR ? 1 : 0);
     // ---- O^T += V^T . P^T -----------------------------------------------
-    if constexpr (FP8) {
+    if constexpr (S::WIDE) {
+        // MFMA u of a d tile takes keys 32h + 8u + [0, 8) of lane half h: the
+        // scores 8 (u & 1) .. of score tile u / 2, and the 8 codes of one
+        // transposing read (read map of the FP8 path below).  The four reads
+        // of a d tile are issued one tile ahead; each is widened under the
+        // MFMA of the one before it.
+        v8bf pop[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) pop[u][e] = (__bf16)s[u >> 1][8 * (u & 1) + e];
+        const uint32_t va = L.v_addr[0] + rt_off;
+        v2i x[2][4];
+        auto issue = [&](auto dc) {
+            constexpr int dt = decltype(dc)::value;
+            const uint32_t addr = va ^ ((2 * dt) << 4);
+            x[dt & 1][0] = ds_read_tr8_b64<VBASE + 0 * ROW>(addr);
+            x[dt & 1][1] = ds_read_tr8_b64<VBASE + 32 * ROW>(addr);
+            x[dt & 1][2] = ds_read_tr8_b64<VBASE + 16 * ROW>(addr);
+            x[dt & 1][3] = ds_read_tr8_b64<VBASE + 48 * ROW>(addr);
+        };
+        issue(std::integral_constant<int, 0>{});
+        v4i vop[2];
+        static_for<0, 4 * DT>([&](auto mc) {
+            constexpr int m = decltype(mc)::value, dt = m >> 2, u = m & 3;
+            if constexpr (m == 0) {
+                lds_results_ready(x[0]);
+                vop[0] = e4m3x8_to_bf16x8(x[0][0][0], x[0][0][1]);
+            }
+            if constexpr (u == 0 && dt + 1 < DT) issue(std::integral_constant<int, dt + 1>{});
+            st.o[dt] = mfma_bf16(vop[m & 1], pop[u], st.o[dt]);
+            if constexpr (m + 1 < 4 * DT) {
+                constexpr int dn = (m + 1) >> 2, un = (m + 1) & 3;
+                if constexpr (un == 0) lds_results_ready(x[dn & 1]);
+                vop[(m + 1) & 1] = e4m3x8_to_bf16x8(x[dn & 1][un][0], x[dn & 1][un][1]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    } else if constexpr (FP8) {
         v8i pop;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -328,8 +353,7 @@ __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off
             for (int k = 0; k < 2; ++k) {
                 const v8i aop = {cur[4 * k][0],     cur[4 * k][1],     cur[4 * k + 1][0], cur[4 * k + 1][1],
                                  cur[4 * k + 2][0], cur[4 * k + 2][1], cur[4 * k + 3][0], cur[4 * k + 3][1]};
-                st.o[2 * pair + k] =
-                    __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aop, pop, st.o[2 * pair + k], 0, 0, 0, 0, 0, 0);
+                st.o[2 * pair + k] = mfma_e4m3(aop, pop, st.o[2 * pair + k]);
             }
         }
         // All 4 row-sum registers stay allocated until here: the inline-asm
@@ -353,7 +377,7 @@ __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off
         // The second buffer of a 32 KB tile lies beyond the 16-bit immediate:
         // its 64 KB part goes into the address.
         constexpr uint32_t VHI = VBASE & ~0xFFFFu;
-        if constexpr (S::PAIR) {
+        if constexpr (S::PAIR_HALVES) {
             // One wave's 32 keys: per d tile two MFMAs (keys 0-15, 16-31 of
             // its half), each operand's two reads issued one MFMA ahead (two
             // 4-register buffers: this mode has no registers for more).
@@ -408,46 +432,49 @@ __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off
     }
 }
 
-// Wait for tile `cur` (in BUF), start the prefetch of `nxt` into the other
-// buffer, then compute `cur`.
-// PAIR (double-buffered): BUF is 0 and rbuf the buffer of `cur`, so that
-// the walk has one loop body (two bodies made the register allocator keep
-// copies of O^T across them and spill).
+// Wait for the step's tiles `cur` (in BUF; TILES of them, the second possibly
+// past the last), start the prefetch of `nxt` into the other buffer, then
+// compute this wave's tile of `cur`.
+// PAIR: BUF is 0 and rbuf the buffer of `cur`, so that the walk has one loop
+// body (two bodies made the register allocator keep copies of O^T across
+// them and spill).
 template <class S, int BUF, bool CAUSAL>
-__device__ __forceinline__ void tile_step(const FwdArgs& a, const TileCursor& cur, const TileCursor& nxt,
-                                          uint8_t* lds, int wave, int tid, int h, const LaneMap<S>& L,
-                                          const QOperand<S> (&qop)[S::QK], float cscale, SoftmaxState<S>& st,
-                                          int row_limit, int first_key, int rbuf) {
-    const int valid = min(kKeyTile, cur.n - cur.base);
-    const uint32_t rt_off = S::PAIR && S::NBUF == 2 ? rbuf * 2 * S::TILE : 0;
-    uint8_t* const lds_v = lds + BUF * 2 * S::TILE + rt_off + S::TILE;
-    if constexpr (S::NBUF == 2) {
-        wait_vmem();      // this wave's loads of the current tile have landed
-        __syncthreads();  // ... and every wave's; the other buffer is free
-        if (nxt.e < a.num_entries) {
-            if constexpr (S::PAIR)
-                stage_tile_async<S, 0>(a, nxt, lds + (rt_off ^ (2 * S::TILE)), wave, L);
-            else
-                stage_tile_async<S, BUF ^ 1>(a, nxt, lds, wave, L);
+__device__ __forceinline__ void tile_step(const FwdArgs& a, const TileCursor (&cur)[S::TILES],
+                                          const TileCursor (&nxt)[S::TILES], uint8_t* lds, int wave, int tid, int h,
+                                          const LaneMap<S>& L, const QOperand<S> (&qop)[S::QK],
+                                          float cscale, SoftmaxState<S>& st, int row_limit, int kh, int rbuf) {
+    const uint32_t rt_off = S::PAIR ? rbuf * S::BUFFER : 0;
+    uint8_t* const buf = lds + BUF * S::BUFFER + rt_off;
+    int valid[S::TILES];
+    bool partial = false;
+#pragma unroll
+    for (int i = 0; i < S::TILES; ++i) {
+        valid[i] = min(kKeyTile, cur[i].n - cur[i].base);  // 0 past the last tile
+        partial |= valid[i] < kKeyTile && (S::TILES == 1 || valid[i] > 0);
+    }
+    wait_vmem();      // this wave's loads of the current tiles have landed
+    __syncthreads();  // ... and every wave's; the other buffer is free
+#pragma unroll
+    for (int i = 0; i < S::TILES; ++i)
+        if (nxt[i].e < a.num_entries) {
+            uint8_t* const other = lds + (S::PAIR ? rt_off ^ S::BUFFER : (BUF ^ 1) * S::BUFFER);
+            stage_tile_async<S>(a, nxt[i], other + i * 2 * S::TILE, wave, L);
         }
-        if (valid < kKeyTile) {
-            zero_masked_v<S>(lds_v, valid, tid);
-            __syncthreads();
-        }
-    } else {
-        __syncthreads();  // previous tile fully consumed
-        if constexpr (S::WIDEN) {
-            stage_tile_sync<S>(a, cur, valid, lds, tid);
-        } else {
-            stage_tile_async<S, 0>(a, cur, lds, wave, L);
-            wait_vmem();
-            __syncthreads();
-            if (valid < kKeyTile) zero_masked_v<S>(lds_v, valid, tid);
-        }
+    if (partial) {
+#pragma unroll
+        for (int i = 0; i < S::TILES; ++i)
+            if (S::TILES == 1 || valid[i] > 0) zero_masked_v<S>(buf + i * 2 * S::TILE + S::TILE, valid[i], tid);
         __syncthreads();
     }
-    compute_tile<S, BUF, CAUSAL>(lds, rt_off, (CAUSAL ? min(valid, row_limit - cur.base) : valid) - first_key, qop,
-                                 cscale, L, h, st);
+    if constexpr (S::TILES == 2) {
+        const int v = kh ? valid[1] : valid[0];
+        if (v > 0) compute_tile<S, BUF, CAUSAL>(lds, rt_off + kh * 2 * S::TILE, v, qop, cscale, L, h, st);
+    } else {
+        const int first_key = S::PAIR ? 32 * kh : 0;
+        compute_tile<S, BUF, CAUSAL>(lds, rt_off,
+                                     (CAUSAL ? min(valid[0], row_limit - cur[0].base) : valid[0]) - first_key, qop,
+                                     cscale, L, h, st);
+    }
 }
 
 // Query row of lane j of the wave in 32-row slot pw: its index among the
@@ -597,7 +624,7 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // PAIR: waves w and w + 4 (one SIMD) share 32 rows; wave w + 4 takes the
-    // tiles' keys 32..63
+    // tiles' keys 32..63 (e4m3 cache: every second tile)
     const int pw = S::PAIR ? wave & (kWaves - 1) : wave;  // the wave's 32-row slot
     const int kh = S::PAIR ? wave / kWaves : 0;           // its key half
     const int j = lane & 31;  // query column of the score tile / A-operand row
@@ -611,6 +638,7 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
     const uint8_t* const qrow = a.q + qr.off;
 
     // ---- Q^T operand (register resident for the whole history) ------------
+    constexpr bool F8 = S::F8;
     QOperand<S> qop[QK];
     float cscale;
     if constexpr (FP8) {
@@ -650,11 +678,12 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
         }
         cscale = sigma * a.score_scale;
     } else {
-        // lane (j, h) holds d = 16c + 8h + [0, 8) of its row.
+        // lane (j, h) holds d = 16c + 8h + [0, 8) of its row (WIDE: 32 (c / 2)
+        // + 16h + 8 (c % 2) + [0, 8), the halves of its 16-code K chunks).
 #pragma unroll
         for (int c = 0; c < QK; ++c) {
-            const v4i raw = *(const v4i*)(qrow + (16 * c + 8 * h) * 2);
-            qop[c] = __builtin_bit_cast(v8bf, raw);
+            const int d = S::WIDE ? 32 * (c >> 1) + 16 * h + 8 * (c & 1) : 16 * c + 8 * h;
+            qop[c] = __builtin_bit_cast(v8bf, *(const v4i*)(qrow + d * 2));
         }
         cscale = a.score_scale;
     }
@@ -664,14 +693,15 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
     // lies below ROW, so XOR-ing a constant into the chunk field is one v_xor.
     LaneMap<S> L;
     {
-        const int row = lds_row<FP8>(key_of_row<FP8>(0, j));
+        const int row = lds_row<F8>(key_of_row<F8>(0, j));
         const int first_chunk = FP8 ? 2 * h : h;
-        L.k_addr = row * ROW + ((first_chunk ^ chunk_swizzle<FP8, CHUNKS>(row)) << 4) + kh * S::K_T1_ROWS * ROW;
+        L.k_addr = row * ROW + ((first_chunk ^ chunk_swizzle<F8, CHUNKS>(row)) << 4) +
+                   (S::PAIR_HALVES ? kh * S::K_T1_ROWS * ROW : 0);
     }
-    if constexpr (FP8) {
+    if constexpr (F8) {
         // key 32*(grp>>1) + (gl>>1) (+ 8s for the other reads) -> row below
-        const int row = lds_row<FP8>(32 * (grp >> 1) + (gl >> 1));
-        L.v_addr[0] = lds_address(lds) + row * ROW + (((grp & 1) ^ chunk_swizzle_v<FP8, CHUNKS>(row)) << 4) +
+        const int row = lds_row<F8>(32 * (grp >> 1) + (gl >> 1));
+        L.v_addr[0] = lds_address(lds) + row * ROW + (((grp & 1) ^ chunk_swizzle_v<F8, CHUNKS>(row)) << 4) +
                       8 * (gl & 1);
         L.rsel = ((lane ^ (lane >> 2)) & 4) ? 0 : 0x38383838;
     } else {
@@ -679,17 +709,16 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
         for (int s2 = 0; s2 < 2; ++s2) {
             const int vkey = 8 * (grp >> 1) + 4 * s2 + (gl >> 2);  // + 16u + 32t: same swizzle
             const int dbyte = 2 * (16 * (grp & 1) + 4 * (gl & 3));
-            L.v_addr[s2] = lds_address(lds) + vkey * ROW + (((dbyte >> 4) ^ chunk_swizzle_v<FP8, CHUNKS>(vkey)) << 4) +
+            L.v_addr[s2] = lds_address(lds) + vkey * ROW + (((dbyte >> 4) ^ chunk_swizzle_v<F8, CHUNKS>(vkey)) << 4) +
                            (dbyte & 15) + kh * 32 * ROW;
         }
     }
-#pragma unroll
-    for (int i = 0; i < (S::DMA_SPLIT ? S::DMA_PER_WAVE : 1); ++i) {
-        const int byte = (S::WAVES * i + wave) * 1024 + lane * 16;
+    {
+        const int byte = wave * 1024 + lane * 16;
         const int row = byte / ROW;
         const int pos = (byte % ROW) / 16;
-        L.dma_off[i] = lds_row<FP8>(row) * S::GROW + (pos ^ chunk_swizzle<FP8, CHUNKS>(row)) * 16;
-        L.dma_off_v[i] = lds_row<FP8>(row) * S::GROW + (pos ^ chunk_swizzle_v<FP8, CHUNKS>(row)) * 16;
+        L.dma_off = lds_row<F8>(row) * ROW + (pos ^ chunk_swizzle<F8, CHUNKS>(row)) * 16;
+        L.dma_off_v = lds_row<F8>(row) * ROW + (pos ^ chunk_swizzle_v<F8, CHUNKS>(row)) * 16;
     }
 
     // ---- walk the block table -----------------------------------------------
@@ -728,35 +757,44 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
         }
     };
 
-    TileCursor cur;
-    if (FIXUP && sparse)
-        cur = range_first;
-    else
-        cur = advance(TileCursor{entry_begin - 1, 0, 0, 0});
-    if constexpr (S::NBUF == 2) {
-        if (cur.e < a.num_entries) stage_tile_async<S, 0>(a, cur, lds, wave, L);
+    // the next step's tiles after `last`
+    auto next_step = [&](TileCursor last, TileCursor (&t)[S::TILES]) {
+#pragma unroll
+        for (int i = 0; i < S::TILES; ++i) t[i] = last = advance(last);
+    };
+    TileCursor cur[S::TILES], nxt[S::TILES];
+    if (FIXUP && sparse) {
+        cur[0] = range_first;
+        if constexpr (S::TILES == 2) cur[1] = advance(cur[0]);
+    } else {
+        next_step(TileCursor{entry_begin - 1, 0, 0, 0}, cur);
     }
-    if constexpr (S::PAIR && S::NBUF == 2) {
-        for (int rbuf = 0; cur.e < a.num_entries; rbuf ^= 1) {
-            const TileCursor nxt = advance(cur);
-            tile_step<S, 0, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, 32 * kh, rbuf);
-            cur = nxt;
+#pragma unroll
+    for (int i = 0; i < S::TILES; ++i)
+        if (cur[i].e < a.num_entries) stage_tile_async<S>(a, cur[i], lds + i * 2 * S::TILE, wave, L);
+    auto take_next = [&] {
+#pragma unroll
+        for (int i = 0; i < S::TILES; ++i) cur[i] = nxt[i];
+    };
+    if constexpr (S::PAIR) {
+        for (int rbuf = 0; cur[0].e < a.num_entries; rbuf ^= 1) {
+            next_step(cur[S::TILES - 1], nxt);
+            tile_step<S, 0, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, kh, rbuf);
+            take_next();
         }
     } else {
-        while (cur.e < a.num_entries) {
-            TileCursor nxt = advance(cur);
-            tile_step<S, 0, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, 32 * kh, 0);
-            cur = nxt;
-            if constexpr (S::NBUF == 2) {
-                if (cur.e >= a.num_entries) break;
-                nxt = advance(cur);
-                tile_step<S, 1, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, 32 * kh, 0);
-                cur = nxt;
-            }
+        while (cur[0].e < a.num_entries) {
+            next_step(cur[0], nxt);
+            tile_step<S, 0, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, kh, 0);
+            take_next();
+            if (cur[0].e >= a.num_entries) break;
+            next_step(cur[0], nxt);
+            tile_step<S, 1, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, kh, 0);
+            take_next();
         }
     }
 
-    // ---- PAIR: the key halves' results meet in the first wave of the pair --
+    // ---- PAIR: the two waves' results meet in the first wave of the pair ----
     if constexpr (S::PAIR) {
         // O^T as [pair][register quad][lane] float4s (conflict-free), m and
         // this lane half's l beside; (m, l) = (-1e30, 0) for a half that saw
