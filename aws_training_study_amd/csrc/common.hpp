@@ -95,6 +95,7 @@ struct FwdArgs {
 // order — a row's fixup result does not depend on the rows gathered with
 // it.  Head h's rows form ceil([h] / 128) groups of 128, numbered head by
 // head.
+constexpr int kGuardMaxHeads = 64;  // KV heads a plan handles (the guarded launch is refused beyond)
 __host__ __device__ __forceinline__ int guard_list_offset(int num_kv_heads) { return (num_kv_heads + 3) / 4 * 4; }
 __host__ __device__ __forceinline__ int guard_head_segment(int rows_per_head) {
     return (rows_per_head + kRowsPerGroup - 1) / kRowsPerGroup * kRowsPerGroup;
@@ -276,10 +277,13 @@ __device__ __forceinline__ int chunk_swizzle_v(int row) {
 // 64 SGPRs live at once), which pushes the loop's scalar state into VGPR
 // lanes; this form needs no SGPR beyond vcc.  (-inf comes from a VGPR: vcc
 // and a literal together exceed the one scalar operand a VALU op may read.)
+// s_nop 1: the two wait states between a VALU write of vcc and a VALU read,
+// which the compiler does not insert inside asm.
 template <int K>
 __device__ __forceinline__ float mask_key_at_or_past(float s, int lim, float ninf) {
     static_assert(K >= 0 && K <= 64, "K must be an inline constant");
     asm("v_cmp_lt_i32_e32 vcc, %1, %2\n\t"
+        "s_nop 1\n\t"
         "v_cndmask_b32_e32 %0, %3, %0, vcc"
         : "+v"(s)
         : "i"(K), "v"(lim), "v"(ninf)

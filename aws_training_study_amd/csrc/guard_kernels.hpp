@@ -31,8 +31,6 @@
 
 namespace pcpa {
 
-// KV heads a guard plan handles (the guarded launch is refused beyond).
-constexpr int kGuardMaxHeads = 64;
 // Capacity of the sparse partials, in query rows over all history ranges:
 // [ranges, groups * 128] FP32 rows of D + 1 values (34 MB at head_dim 256).
 constexpr int64_t kGuardPartialRows = 32768;

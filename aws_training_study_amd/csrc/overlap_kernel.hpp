@@ -57,7 +57,7 @@ __device__ __forceinline__ void mask_tail(v16f (&s)[2], int valid, int h) {
 
 
 // ============================================================================
-// FP8 kernel with an in-wave MFMA/softmax overlap (head_dim 128 and 256).
+// FP8 kernel with an in-wave MFMA/softmax overlap.
 //
 // gfx950 overlaps an MFMA with independent VALU work of the same wave, but a
 // single wave per SIMD issues too slowly to keep the matrix core busy.  So
@@ -87,14 +87,16 @@ __device__ __forceinline__ void mask_tail(v16f (&s)[2], int valid, int h) {
 // ============================================================================
 namespace ovl {
 
-constexpr int kWaves = 8;
-constexpr int kThreads = 64 * kWaves;
-constexpr int kRowsPerGroup = kWaves * 32;
 constexpr int kStages = 4;
+constexpr int kDmaWaves = 4;  // waves of a workgroup that issue its LDS-DMA
+
+// Query rows and threads of a workgroup of `waves` waves.
+constexpr int rows_per_group(int waves) { return waves * 32; }
+constexpr int threads(int waves) { return waves * 64; }
 
 template <int D>
 struct Shape {
-    static_assert(D == 128 || D == 256, "overlap kernel covers head_dim 128 and 256");
+    static_assert(D == 64 || D == 128 || D == 256, "head_dim 64, 128 or 256");
     static constexpr int ROW = D;            // e4m3 bytes of one key row
     static constexpr int CHUNKS = D / 16;
     static constexpr int TILE = kKeyTile * ROW;
@@ -106,21 +108,21 @@ struct Shape {
     static constexpr int pv_begin(int i) {
         constexpr int b256[] = {0, 4, 6, 7, 8, 9, 10, 11, 14};
         constexpr int b128[] = {0, 5, 8, 11, 14};
-        return D == 256 ? b256[i] : b128[i];
+        constexpr int b64[] = {0, 7, 14};
+        return D == 256 ? b256[i] : D == 128 ? b128[i] : b64[i];
     }
 };
 
-// Who moves the K and V tiles: the last WAVES = kWaves / 2 waves of the
-// workgroup, the group that runs PV first (one wave per SIMD), issue the
-// LDS-DMA of every K and V tile and each waits for its own blocks; the
-// barrier after the waits publishes them to all waves (about 1% faster than
-// all eight waves issuing).
-template <int D, int WAVES>
+// Who moves the K and V tiles: the last kDmaWaves waves of the workgroup (of
+// eight, the group that runs PV first, one wave per SIMD; about 1% faster than
+// all eight waves issuing).  They issue the LDS-DMA of every K and V tile and
+// each waits for its own blocks; the barrier after the waits publishes them to
+// all waves.
+template <int D>
 struct DmaPlan {
-    static_assert(WAVES == kWaves / 2, "the PV-first group issues all DMA");
     static constexpr int ROW = D;
-    static constexpr int DPW = kKeyTile * ROW / 1024 / WAVES;  // 1 KB blocks per wave per K (or V) tile
-    static constexpr int STRIDE = WAVES * 1024;                // LDS bytes between a wave's blocks
+    static constexpr int DPW = kKeyTile * ROW / 1024 / kDmaWaves;  // 1 KB blocks per wave per K (or V) tile
+    static constexpr int STRIDE = kDmaWaves * 1024;                // LDS bytes between a wave's blocks
     // A wave's block i lands i * BLOCK_ROWS LDS rows after its block 0
     // (rows < BLOCK_ROWS).  lds_row permutes row bits, so block i holds the
     // keys lds_row(i * BLOCK_ROWS) further on; a multiple of 16 rows keeps
@@ -132,8 +134,8 @@ struct DmaPlan {
     static constexpr int offset(int i) { return lds_row<true>(i * BLOCK_ROWS) * ROW; }
     static constexpr int MID = offset(DPW - 1) / 2;
     static_assert(MID < 4096, "DMA block offsets must fit the immediate");
-    __device__ static bool issues(int wave) { return wave >= kWaves - WAVES; }
-    __device__ static int block(int wave) { return wave - (kWaves - WAVES); }
+    __device__ static bool issues(int wave, int waves) { return wave >= waves - kDmaWaves; }
+    __device__ static int block(int wave) { return wave % kDmaWaves; }
 };
 
 struct Lanes {
@@ -182,6 +184,10 @@ struct SoftmaxRow {
 // 362 < 448) and rescale factor; 5-12: four probabilities each, one dword
 // of P; 13: reference update.  The row sum is taken from P by an MFMA.
 //
+// TRAIL false: the reference max stays until a tile's max exceeds it by more
+// than 2.5 and then becomes that max (the rule of history_fwd_kernel, whose
+// e4m3 codes head_dim 64 and 128 keep).
+//
 // FAST: P = 2^x (x = s * cscale + 6 - m_use) is produced directly as its
 // e4m3 code round(8x + 56), clamped to [0, 255] by v_cvt_pk_u8_f32.  For
 // x = n + f that code decodes to 2^n (1 + f) rounded to 3 mantissa bits:
@@ -190,7 +196,7 @@ struct SoftmaxRow {
 // rounding step of P itself.  Codes below 8 are the e4m3 subnormals of
 // values under 2^-6, i.e. under 2^-14 of the tile max.  Otherwise P =
 // v_exp_f32 rounded by v_cvt_pk_fp8_f32.
-template <int K, bool FAST>
+template <int K, bool FAST, bool TRAIL>
 __device__ __forceinline__ void softmax_slice(const v16f (&s)[2], v8i& p, SoftmaxRow& sm) {
     if constexpr (K < 4) {
         constexpr int t = K >> 1, r = 8 * (K & 1);
@@ -202,7 +208,7 @@ __device__ __forceinline__ void softmax_slice(const v16f (&s)[2], v8i& p, Softma
         pin(sm.mx);
     } else if constexpr (K == 4) {
         const float mxs = halves_max(sm.mx) * sm.cscale;
-        sm.m_use = fmaxf(sm.m, mxs - 2.5f);
+        sm.m_use = TRAIL ? fmaxf(sm.m, mxs - 2.5f) : (mxs > sm.m + 2.5f ? mxs : sm.m);
         sm.alpha = __builtin_amdgcn_exp2f(sm.m - sm.m_use);
         // FAST: 8x + 56 = s * 8 cscale + (8 (6 - m_use) + 56)
         sm.shift = FAST ? fmaf(-8.f, sm.m_use, 8.f * kPBiasLog2 + 56.f) : kPBiasLog2 - sm.m_use;
@@ -235,11 +241,11 @@ __device__ __forceinline__ void softmax_slice(const v16f (&s)[2], v8i& p, Softma
     }
 }
 
-template <int LO, int HI, bool FAST>
+template <int LO, int HI, bool FAST, bool TRAIL>
 __device__ __forceinline__ void softmax_slices(const v16f (&s)[2], v8i& p, SoftmaxRow& sm) {
     if constexpr (LO < HI) {
-        softmax_slice<LO, FAST>(s, p, sm);
-        softmax_slices<LO + 1, HI, FAST>(s, p, sm);
+        softmax_slice<LO, FAST, TRAIL>(s, p, sm);
+        softmax_slices<LO + 1, HI, FAST, TRAIL>(s, p, sm);
     }
 }
 
@@ -277,6 +283,22 @@ __device__ __forceinline__ const uint8_t* k_tile(const FwdArgs& a, const TileCur
 template <class S>
 __device__ __forceinline__ const uint8_t* v_tile(const FwdArgs& a, const TileCursor& c) {
     return k_tile<S>(a, c) + (int64_t)a.num_kv_heads * a.head_stride;
+}
+
+// A wave-uniform pointer, moved to SGPRs: the compiler forms the tile
+// addresses of some four-wave instantiations with VALU instructions and then
+// passes the VGPRs to the LDS-DMA's SGPR operand (the builtin folds away).
+__device__ __forceinline__ const uint8_t* to_sgprs(const uint8_t* p) {
+    const uint64_t x = (uint64_t)p;
+    uint32_t lo, hi;
+    // Wait states that the compiler would insert around the instructions but
+    // not around the asm: s_nop 1 (a VGPR written by VALU needs one before
+    // v_readfirstlane reads it), s_nop 4 (a VALU-written SGPR needs five
+    // before a VMEM read).
+    asm volatile("s_nop 1\n\tv_readfirstlane_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3\n\ts_nop 4"
+                 : "=&s"(lo), "=&s"(hi)
+                 : "v"((uint32_t)x), "v"((uint32_t)(x >> 32)));
+    return (const uint8_t*)(((uint64_t)hi << 32) | lo);
 }
 
 // Issue the K tile of cursor c into K stage st (lds: LDS address of the
@@ -412,7 +434,7 @@ __device__ __forceinline__ void pv_half(uint32_t v_addr, v2i (&xv0)[4], v16f (&o
         const v8i vop = {x[0][0], x[0][1], x[1][0], x[1][1], x[2][0], x[2][1], x[3][0], x[3][1]};
         o[dt] = mfma_e4m3(vop, p_old, o[dt]);
         after_mfma(dc);
-        softmax_slices<S::pv_begin(dt), S::pv_begin(dt + 1), FAST>(s, p_new, sm);
+        softmax_slices<S::pv_begin(dt), S::pv_begin(dt + 1), FAST, D == 256>(s, p_new, sm);
         __builtin_amdgcn_sched_barrier(0);
     });
     // O^T gained P_old's tile; both O^T and l move to the new reference (l
@@ -424,8 +446,9 @@ __device__ __forceinline__ void pv_half(uint32_t v_addr, v2i (&xv0)[4], v16f (&o
     }
 }
 
-// Iteration j, J4 = j mod 4; LATE: waves 4-7 (PV half first, one tile behind).
-template <int D, int J4, bool LATE, bool FAST, int DMAW>
+// Iteration j, J4 = j mod 4; LATE: the waves that run the PV half first, one
+// tile behind.  DMA: the wave issues LDS-DMA.
+template <int D, int J4, bool LATE, bool FAST, bool DMA>
 __device__ __forceinline__ void iteration(const FwdArgs& a, uint8_t* lds, int wave, int h, const Lanes& L,
                                           const v8i (&q)[Shape<D>::QK], v16f (&s)[2], v8i (&pbuf)[2],
                                           v16f (&o)[Shape<D>::DT], SoftmaxRow& sm, Cursors& cs, int head,
@@ -437,8 +460,8 @@ __device__ __forceinline__ void iteration(const FwdArgs& a, uint8_t* lds, int wa
     // Loads issued one iteration ago may be pending: V(j) and K(j+1) (a
     // phantom K tile is loaded too).  Each wave that issues DMA waits for its own blocks; the
     // barrier then publishes all of them.
-    using P = DmaPlan<D, DMAW>;
-    if constexpr (LATE) wait_vmem_le<2 * P::DPW>();
+    using P = DmaPlan<D>;
+    if constexpr (DMA) wait_vmem_le<2 * P::DPW>();
     __builtin_amdgcn_s_barrier();
     // The wave offset and operand bases
     // are made opaque so that the DMA destinations and operand addresses are
@@ -446,39 +469,53 @@ __device__ __forceinline__ void iteration(const FwdArgs& a, uint8_t* lds, int wa
     int wave_off = P::block(wave) * 1024;
     uint32_t k_addr = L.k_addr, v_addr = L.v_addr;
     asm volatile("" : "+s"(wave_off), "+v"(k_addr), "+v"(v_addr));
+    // The DMA of K(j+2) and V(j+1) is spread over the issuing waves' PV half,
+    // one block per PV MFMA (more where a tile has more blocks than that): K
+    // first, then V (a V tile with masked rows, rare, is issued before the
+    // half).  K stage (j+2) % 4 and V stage (j+1) % 4 were last read in
+    // iteration j-1, before this iteration's barrier.
+    const uint32_t lds_u = lds_address(lds);
+    const bool v_real = is_real(a, cs.c1);
+    const int v_valid = v_real ? cs.c1.n - cs.c1.base : 0;
+    const uint8_t* ktile = k_tile<S>(a, cs.c2);
+    const uint32_t kdst = lds_u + ((J4 + 2) % kStages) * S::TILE + wave_off;
+    const uint8_t* vtile = v_tile<S>(a, cs.c1);
+    if constexpr (DMA && !LATE) {
+        ktile = to_sgprs(ktile);
+        vtile = to_sgprs(vtile);
+    }
+    const uint32_t vdst = lds_u + S::RING + ((J4 + 1) % kStages) * S::TILE + wave_off;
+    auto dma_step = [&](auto dc) {
+        if constexpr (DMA) {
+            constexpr int per = (2 * P::DPW + S::DT - 1) / S::DT, first = decltype(dc)::value * per;
+            static_for<first, (first + per < 2 * P::DPW ? first + per : 2 * P::DPW)>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (i < P::DPW) {
+                    dma_block<P, i>(ktile, L.dma_k, kdst);
+                } else {
+                    if (v_valid >= kKeyTile) dma_block<P, i - P::DPW>(vtile, L.dma_v, vdst);
+                }
+            });
+        }
+    };
+    auto dma_partial = [&] {
+        if constexpr (DMA)
+            if (v_valid < kKeyTile)
+                load_v_partial<S, P>(a, cs.c1, lds_u, (J4 + 1) % kStages, wave_off, L.dma_v, v_valid);
+    };
     if constexpr (!LATE) {
         // S(j), then PV(j-1) beside softmax(j)
         constexpr int VST = (J4 + 3) % kStages;
         s_half<D, KST, true, VST>(k_addr, v_addr, q, s, xv, pbuf[J4 & 1], sm, L.rsel);
-        pv_half<D, VST, true, FAST>(v_addr, xv, o, pbuf[(J4 + 1) & 1], s, pbuf[J4 & 1], sm,
-                              cs.k0, h, [](auto) {});
+        dma_partial();
+        pv_half<D, VST, true, FAST>(v_addr, xv, o, pbuf[(J4 + 1) & 1], s, pbuf[J4 & 1], sm, cs.k0, h, dma_step);
     } else {
         // PV(j-2) beside softmax(j-1), then S(j).  The first V-operand read
         // of PV(j-2) was issued at the end of the previous iteration's S half
         // (V(j-2) landed before the previous barrier), so it is in flight
         // across the barrier; this S half issues the one for PV(j-1).
         constexpr int VST = (J4 + 2) % kStages;
-        // This group's DMA of K(j+2) and V(j+1) is spread over its PV half,
-        // one block per PV MFMA: K after the first DPW, V after the next DPW
-        // (a V tile with masked rows, rare, is issued before the half).  K
-        // stage (j+2) % 4 and V stage (j+1) % 4 were last read in iteration
-        // j-1, before this iteration's barrier.
-        const uint32_t lds_u = lds_address(lds);
-        const bool v_real = is_real(a, cs.c1);
-        const int v_valid = v_real ? cs.c1.n - cs.c1.base : 0;
-        if (v_valid < kKeyTile) load_v_partial<S, P>(a, cs.c1, lds_u, (J4 + 1) % kStages, wave_off, L.dma_v, v_valid);
-        const uint8_t* const ktile = k_tile<S>(a, cs.c2);
-        const uint32_t kdst = lds_u + ((J4 + 2) % kStages) * S::TILE + wave_off;
-        const uint8_t* const vtile = v_tile<S>(a, cs.c1);
-        const uint32_t vdst = lds_u + S::RING + ((J4 + 1) % kStages) * S::TILE + wave_off;
-        auto dma_step = [&](auto dc) {
-            constexpr int i = decltype(dc)::value;
-            if constexpr (i < P::DPW) {
-                dma_block<P, i>(ktile, L.dma_k, kdst);
-            } else if constexpr (i < 2 * P::DPW) {
-                if (v_valid >= kKeyTile) dma_block<P, i - P::DPW>(vtile, L.dma_v, vdst);
-            }
-        };
+        dma_partial();
         // this half carries the group's LDS-DMA issue and softmax VALU work;
         // issuing it ahead of the other wave on the SIMD (whose score MFMAs
         // queue on the matrix core anyway) measured 0.65% faster on the
@@ -497,27 +534,31 @@ __device__ __forceinline__ void iteration(const FwdArgs& a, uint8_t* lds, int wa
 }
 
 // The loop of one wave group; iteration j runs while j <= T + 1 (T tiles).
-template <int D, bool LATE, bool FAST, int DMAW>
+template <int D, bool LATE, bool FAST, bool DMA>
 __device__ __forceinline__ void walk(const FwdArgs& a, uint8_t* lds, int wave, int h, const Lanes& L,
                                      const v8i (&q)[Shape<D>::QK], v16f (&s)[2], v8i (&pbuf)[2],
                                      v16f (&o)[Shape<D>::DT], SoftmaxRow& sm, Cursors cs, int head) {
     // the first V-operand read of the next PV half (the PV-first waves start
     // with PV(-2): V stage 2, zeros)
     v2i xv[4];
-    if constexpr (LATE) read_v_operand<D, 2>(L.v_addr, xv);
+    if constexpr (LATE) {
+        read_v_operand<D, 2>(L.v_addr, xv);
+        // (landed before the loop: its entry may copy the registers)
+        lds_wait<0>(xv);
+    }
     for (;;) {
         // after iteration j the loop ends if tile j-1 was past the last tile
         bool done = cs.km1 < 0;
-        iteration<D, 0, LATE, FAST, DMAW>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
+        iteration<D, 0, LATE, FAST, DMA>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
         if (done) break;
         done = cs.km1 < 0;
-        iteration<D, 1, LATE, FAST, DMAW>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
+        iteration<D, 1, LATE, FAST, DMA>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
         if (done) break;
         done = cs.km1 < 0;
-        iteration<D, 2, LATE, FAST, DMAW>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
+        iteration<D, 2, LATE, FAST, DMA>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
         if (done) break;
         done = cs.km1 < 0;
-        iteration<D, 3, LATE, FAST, DMAW>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
+        iteration<D, 3, LATE, FAST, DMA>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head, xv);
         if (done) break;
     }
     // the PV-first waves' last S half read an operand of a PV half that does
@@ -544,13 +585,14 @@ __device__ __forceinline__ int64_t query_row_offset(const FwdArgs& a, int row, i
 // SPLIT: the workgroup walks only its split's share of the table entries
 // and writes a normalised FP32 partial output and log-sum-exp (merged by
 // merge_splits_kernel).
-template <int D, bool FAST, bool LSE, bool SPLIT = false>
-__global__ void __launch_bounds__(kThreads, 1) history_fwd_overlap(FwdArgs a) {
+// WAVES: 8, staggered in two groups of one wave per SIMD, or 4 (one wave per
+// SIMD, all running S first and all issuing DMA).
+template <int D, bool FAST, bool LSE, bool SPLIT, int WAVES>
+__device__ __forceinline__ void overlap_body(FwdArgs& a, uint8_t* lds) {
     using S = Shape<D>;
     constexpr int QK = S::QK, DT = S::DT, ROW = S::ROW, CHUNKS = S::CHUNKS;
-    constexpr int DMAW = kWaves / 2;
-    using P = DmaPlan<D, DMAW>;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * S::RING];
+    constexpr int kThreads = threads(WAVES), kRowsPerGroup = rows_per_group(WAVES);
+    using P = DmaPlan<D>;
 
     // ---- XCD-aware work mapping (as history_fwd_kernel) ---------------------
     // Items run row tile fastest, so an XCD's workgroups share one (KV head,
@@ -665,17 +707,19 @@ __global__ void __launch_bounds__(kThreads, 1) history_fwd_overlap(FwdArgs a) {
         cs.c1 = next_tile(a, head, first);
         cs.c2 = is_real(a, cs.c1) ? next_tile(a, head, cs.c1) : cs.c1;
         // K(0), then V(0) and K(1) as if requested in iteration -1.
-        if (P::issues(wave)) {
+        if (P::issues(wave, WAVES)) {
             const int wave_off = P::block(wave) * 1024;
             const uint32_t lds_u = lds_address(lds);
             load_k<S, P>(a, first, lds_u, 0, wave_off, L.dma_k);
             load_v<S, P>(a, first, lds_u, 0, wave_off, L.dma_v, true);
             load_k<S, P>(a, cs.c1, lds_u, 1, wave_off, L.dma_k);
         }
-        if (wave < kWaves / 2)
-            walk<D, false, FAST, DMAW>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head);
+        if constexpr (WAVES == 4)
+            walk<D, false, FAST, true>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head);
+        else if (wave < WAVES / 2)
+            walk<D, false, FAST, false>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head);
         else
-            walk<D, true, FAST, DMAW>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head);
+            walk<D, true, FAST, true>(a, lds, wave, h, L, q, s, pbuf, o, sm, cs, head);
     }
 
     // ---- epilogue: O = O^T / l, bf16; log-sum-exp ---------------------------
@@ -697,28 +741,39 @@ __global__ void __launch_bounds__(kThreads, 1) history_fwd_overlap(FwdArgs a) {
     if constexpr (SPLIT) {
         if (row_ok) {
             const int64_t prow = (int64_t)split * a.rows_per_head * a.num_kv_heads + row_off / (D * 2);
-            // fp16 partials of O / l, before the v_scale factor (the merge
-            // applies it): a weighted mean of e4m3 V codes, |O / l| <= 448
-            // whatever v_scale is, so fp16 keeps its relative precision;
-            // half the bytes of fp32 for this kernel to write and the merge
-            // to read
-            const float inv_l = sm.l > 0.f ? 1.f / sm.l : 0.f;
-            _Float16* const po = (_Float16*)a.part_o + prow * D;
+            if constexpr (D == 256) {
+                // fp16 partials of O / l, before the v_scale factor (the merge
+                // applies it): a weighted mean of e4m3 V codes, |O / l| <= 448
+                // whatever v_scale is, so fp16 keeps its relative precision;
+                // half the bytes of fp32 for this kernel to write and the merge
+                // to read
+                const float inv_l = sm.l > 0.f ? 1.f / sm.l : 0.f;
+                _Float16* const po = (_Float16*)a.part_o + prow * D;
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+                for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4) {
-                    const int d = 32 * dt + 8 * r4 + 4 * h;
-                    uint32_t w[2];
+                    for (int r4 = 0; r4 < 4; ++r4) {
+                        const int d = 32 * dt + 8 * r4 + 4 * h;
+                        uint32_t w[2];
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        const _Float16 x0 = (_Float16)(o[dt][4 * r4 + 2 * i] * inv_l);
-                        const _Float16 x1 = (_Float16)(o[dt][4 * r4 + 2 * i + 1] * inv_l);
-                        w[i] = (uint32_t)__builtin_bit_cast(uint16_t, x0) |
-                               ((uint32_t)__builtin_bit_cast(uint16_t, x1) << 16);
+                        for (int i = 0; i < 2; ++i) {
+                            const _Float16 x0 = (_Float16)(o[dt][4 * r4 + 2 * i] * inv_l);
+                            const _Float16 x1 = (_Float16)(o[dt][4 * r4 + 2 * i + 1] * inv_l);
+                            w[i] = (uint32_t)__builtin_bit_cast(uint16_t, x0) |
+                                   ((uint32_t)__builtin_bit_cast(uint16_t, x1) << 16);
+                        }
+                        *(v2i*)(po + d) = v2i{(int)w[0], (int)w[1]};
                     }
-                    *(v2i*)(po + d) = v2i{(int)w[0], (int)w[1]};
-                }
+            } else {
+                float* const po = a.part_o + prow * D;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int r4 = 0; r4 < 4; ++r4)
+                        *(v4f*)(po + 32 * dt + 8 * r4 + 4 * h) =
+                            v4f{o[dt][4 * r4] * scale, o[dt][4 * r4 + 1] * scale, o[dt][4 * r4 + 2] * scale,
+                                o[dt][4 * r4 + 3] * scale};
+            }
             if (h == 0) {
                 a.part_lse[prow] = lse;
                 if (a.part_m) a.part_m[prow] = sm.m;
@@ -755,6 +810,28 @@ __global__ void __launch_bounds__(kThreads, 1) history_fwd_overlap(FwdArgs a) {
     }
 }
 
+// Eight waves, 256 rows, at head_dim 256.
+template <int D, bool FAST, bool LSE, bool SPLIT = false>
+__global__ void __launch_bounds__(threads(8), 1) history_fwd_overlap(FwdArgs a) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * Shape<D>::RING];
+    overlap_body<D, FAST, LSE, SPLIT, 8>(a, lds);
+}
+
+// Any head dim and workgroup size.  The LDS (lds_bytes(D)) is dynamic so that
+// the compiler does not see that it leaves a CU one workgroup: it then keeps
+// to 256 VGPRs a wave.  With the four waves of a static 128 KB workgroup it
+// took 368 registers, the accumulators in AGPRs, and copied the scores out of
+// them (head_dim 256, 64 row tiles x 2 ranges of 16 key tiles: 46.4 us against
+// 34; workgroups of 256 rows 44.6).  head_dim 128 and 64 run here rather than
+// on the tile kernel because a wave's softmax issues under its own PV MFMAs:
+// 64 x 8 heads at head_dim 128, 2048 x 30011, 1218 -> 1165 us a call.
+template <int D, bool FAST, bool LSE, bool SPLIT, int WAVES>
+__global__ void __launch_bounds__(threads(WAVES), 8 / WAVES) history_fwd_overlap_waves(FwdArgs a) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t dynamic_lds[];
+    overlap_body<D, FAST, LSE, SPLIT, WAVES>(a, dynamic_lds);
+}
+constexpr int lds_bytes(int d) { return 2 * kStages * kKeyTile * d; }
+
 }  // namespace ovl
 
 // Merge of split partial outputs by log-sum-exp: one thread per (row, 8
@@ -774,20 +851,24 @@ __global__ void __launch_bounds__(kThreads, 1) history_fwd_overlap(FwdArgs a) {
 // memory instead of three (2-split 16-rank workload: 0.1761 against 0.1792
 // ms per call; 8-split 4-rank BF16 workload: 0.0124 against 0.0137 ms);
 // NS == 0: any count.
+constexpr int kMergeThreads = 1024;
 template <int NS>
-__global__ void __launch_bounds__(256) merge_splits_kernel(const float* part_o, int part_f16, float part_scale,
+__global__ void __launch_bounds__(kMergeThreads) merge_splits_kernel(const float* part_o, int part_f16, float part_scale,
                                                            const float* part_lse, int splits, int64_t rows, int d_vec8, uint8_t* out,
                                                            float* lse_out,
                                                            const float* part_m, int32_t* guard_plan, GuardShape g,
                                                            float lse_bias, const float* guard_thr) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= rows * d_vec8) return;
-    const int64_t row = idx / d_vec8;
-    const int d0 = (int)(idx - row * d_vec8) * 8;
+    __shared__ int listed[kGuardMaxHeads];
+    const int64_t idx = (int64_t)blockIdx.x * kMergeThreads + threadIdx.x;
+    const bool real = idx < rows * d_vec8;
+    if (!guard_plan && !real) return;
+    const int64_t row = real ? idx / d_vec8 : rows - 1;
+    const int d0 = real ? (int)(idx - row * d_vec8) * 8 : 0;
     const int D = d_vec8 * 8;
     if constexpr (NS > 0) splits = NS;
+    if (guard_plan && threadIdx.x < g.num_kv_heads) listed[threadIdx.x] = 0;
     // the guard's inputs first, so that their loads overlap the partials'
-    const bool guard_lane = guard_plan && d0 == 0;
+    const bool guard_lane = guard_plan && real && d0 == 0;
     int head = 0, head_row = 0;
     float thr = 0.f, m_ref = -INFINITY;
     if (guard_lane) {
@@ -864,13 +945,29 @@ __global__ void __launch_bounds__(256) merge_splits_kernel(const float* part_o, 
         const __bf16 x0 = (__bf16)(acc[2 * i] * inv), x1 = (__bf16)(acc[2 * i + 1] * inv);
         wv[i] = (uint32_t)__builtin_bit_cast(uint16_t, x0) | ((uint32_t)__builtin_bit_cast(uint16_t, x1) << 16);
     }
-    *(v4i*)(out + (row * D + d0) * 2) = v4i{(int)wv[0], (int)wv[1], (int)wv[2], (int)wv[3]};
+    if (real) *(v4i*)(out + (row * D + d0) * 2) = v4i{(int)wv[0], (int)wv[1], (int)wv[2], (int)wv[3]};
     const float lse = wsum > 0.f ? mx + __logf(wsum) : -INFINITY;
-    if (lse_out && d0 == 0) lse_out[row] = lse;
+    if (lse_out && real && d0 == 0) lse_out[row] = lse;
+    if (!guard_plan) return;
+    // The workgroup's rows below their threshold: counted per KV head in LDS,
+    // one device atomic per head that has any (an atomic per wave queued
+    // hundreds of them on a few counters: 8192 rows with 890 listed took 15
+    // us, now 8).
+    bool low = false;
+    int pos = 0;
+    __syncthreads();
     if (guard_lane) {
         const float mass = wsum > 0.f ? __expf(lse + lse_bias - m_ref * kLn2) : 0.f;
-        if (mass < thr) guard_append(guard_plan, g.num_kv_heads, g.rows_per_head, head, head_row);
+        low = mass < thr;
+        if (low) pos = atomicAdd(&listed[head], 1);
     }
+    __syncthreads();
+    if (threadIdx.x < g.num_kv_heads && listed[threadIdx.x] > 0)
+        listed[threadIdx.x] = atomicAdd(&guard_plan[threadIdx.x], listed[threadIdx.x]);
+    __syncthreads();
+    if (low)
+        guard_plan[guard_list_offset(g.num_kv_heads) + head * guard_head_segment(g.rows_per_head) + listed[head] +
+                   pos] = head_row;
 }
 
 }  // namespace pcpa
