@@ -44,7 +44,9 @@ constexpr int64_t kGuardPartialRows = 32768;
 // at once and sums them against its own largest log-sum-exp; the groups'
 // sums meet in LDS, rescaled to the row's largest.  Dense mode: nothing.
 constexpr int kGuardMergeThreads = 256;
-constexpr int kGuardMergeGroups = 512;  // workgroups of guard_merge_kernel
+constexpr int kGuardMergeGroups = 1024;  // workgroups of guard_merge_kernel: rows of a launch that lists
+                                         // thousands are taken in turns (2798 rows x 10 ranges: 512
+                                         // workgroups 9 us slower; idle, no difference)
 constexpr int kGuardMergePer = 8;       // ranges per thread at most
 
 __global__ void __launch_bounds__(kGuardMergeThreads) guard_merge_kernel(const float* part_o, const float* part_lse,

@@ -96,7 +96,7 @@ constexpr int threads(int waves) { return waves * 64; }
 
 template <int D>
 struct Shape {
-    static_assert(D == 64 || D == 128 || D == 256, "head_dim 64, 128 or 256");
+    static_assert(D == 128 || D == 256, "head_dim 128 or 256");
     static constexpr int ROW = D;            // e4m3 bytes of one key row
     static constexpr int CHUNKS = D / 16;
     static constexpr int TILE = kKeyTile * ROW;
@@ -108,8 +108,7 @@ struct Shape {
     static constexpr int pv_begin(int i) {
         constexpr int b256[] = {0, 4, 6, 7, 8, 9, 10, 11, 14};
         constexpr int b128[] = {0, 5, 8, 11, 14};
-        constexpr int b64[] = {0, 7, 14};
-        return D == 256 ? b256[i] : D == 128 ? b128[i] : b64[i];
+        return D == 256 ? b256[i] : b128[i];
     }
 };
 
@@ -184,10 +183,6 @@ struct SoftmaxRow {
 // 362 < 448) and rescale factor; 5-12: four probabilities each, one dword
 // of P; 13: reference update.  The row sum is taken from P by an MFMA.
 //
-// TRAIL false: the reference max stays until a tile's max exceeds it by more
-// than 2.5 and then becomes that max (the rule of history_fwd_kernel, whose
-// e4m3 codes head_dim 64 and 128 keep).
-//
 // FAST: P = 2^x (x = s * cscale + 6 - m_use) is produced directly as its
 // e4m3 code round(8x + 56), clamped to [0, 255] by v_cvt_pk_u8_f32.  For
 // x = n + f that code decodes to 2^n (1 + f) rounded to 3 mantissa bits:
@@ -196,7 +191,7 @@ struct SoftmaxRow {
 // rounding step of P itself.  Codes below 8 are the e4m3 subnormals of
 // values under 2^-6, i.e. under 2^-14 of the tile max.  Otherwise P =
 // v_exp_f32 rounded by v_cvt_pk_fp8_f32.
-template <int K, bool FAST, bool TRAIL>
+template <int K, bool FAST>
 __device__ __forceinline__ void softmax_slice(const v16f (&s)[2], v8i& p, SoftmaxRow& sm) {
     if constexpr (K < 4) {
         constexpr int t = K >> 1, r = 8 * (K & 1);
@@ -208,7 +203,7 @@ __device__ __forceinline__ void softmax_slice(const v16f (&s)[2], v8i& p, Softma
         pin(sm.mx);
     } else if constexpr (K == 4) {
         const float mxs = halves_max(sm.mx) * sm.cscale;
-        sm.m_use = TRAIL ? fmaxf(sm.m, mxs - 2.5f) : (mxs > sm.m + 2.5f ? mxs : sm.m);
+        sm.m_use = fmaxf(sm.m, mxs - 2.5f);
         sm.alpha = __builtin_amdgcn_exp2f(sm.m - sm.m_use);
         // FAST: 8x + 56 = s * 8 cscale + (8 (6 - m_use) + 56)
         sm.shift = FAST ? fmaf(-8.f, sm.m_use, 8.f * kPBiasLog2 + 56.f) : kPBiasLog2 - sm.m_use;
@@ -241,11 +236,11 @@ __device__ __forceinline__ void softmax_slice(const v16f (&s)[2], v8i& p, Softma
     }
 }
 
-template <int LO, int HI, bool FAST, bool TRAIL>
+template <int LO, int HI, bool FAST>
 __device__ __forceinline__ void softmax_slices(const v16f (&s)[2], v8i& p, SoftmaxRow& sm) {
     if constexpr (LO < HI) {
-        softmax_slice<LO, FAST, TRAIL>(s, p, sm);
-        softmax_slices<LO + 1, HI, FAST, TRAIL>(s, p, sm);
+        softmax_slice<LO, FAST>(s, p, sm);
+        softmax_slices<LO + 1, HI, FAST>(s, p, sm);
     }
 }
 
@@ -434,7 +429,7 @@ __device__ __forceinline__ void pv_half(uint32_t v_addr, v2i (&xv0)[4], v16f (&o
         const v8i vop = {x[0][0], x[0][1], x[1][0], x[1][1], x[2][0], x[2][1], x[3][0], x[3][1]};
         o[dt] = mfma_e4m3(vop, p_old, o[dt]);
         after_mfma(dc);
-        softmax_slices<S::pv_begin(dt), S::pv_begin(dt + 1), FAST, D == 256>(s, p_new, sm);
+        softmax_slices<S::pv_begin(dt), S::pv_begin(dt + 1), FAST>(s, p_new, sm);
         __builtin_amdgcn_sched_barrier(0);
     });
     // O^T gained P_old's tile; both O^T and l move to the new reference (l
@@ -470,8 +465,7 @@ __device__ __forceinline__ void iteration(const FwdArgs& a, uint8_t* lds, int wa
     uint32_t k_addr = L.k_addr, v_addr = L.v_addr;
     asm volatile("" : "+s"(wave_off), "+v"(k_addr), "+v"(v_addr));
     // The DMA of K(j+2) and V(j+1) is spread over the issuing waves' PV half,
-    // one block per PV MFMA (more where a tile has more blocks than that): K
-    // first, then V (a V tile with masked rows, rare, is issued before the
+    // one block per PV MFMA: K first, then V (a V tile with masked rows, rare, is issued before the
     // half).  K stage (j+2) % 4 and V stage (j+1) % 4 were last read in
     // iteration j-1, before this iteration's barrier.
     const uint32_t lds_u = lds_address(lds);
@@ -487,15 +481,13 @@ __device__ __forceinline__ void iteration(const FwdArgs& a, uint8_t* lds, int wa
     const uint32_t vdst = lds_u + S::RING + ((J4 + 1) % kStages) * S::TILE + wave_off;
     auto dma_step = [&](auto dc) {
         if constexpr (DMA) {
-            constexpr int per = (2 * P::DPW + S::DT - 1) / S::DT, first = decltype(dc)::value * per;
-            static_for<first, (first + per < 2 * P::DPW ? first + per : 2 * P::DPW)>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                if constexpr (i < P::DPW) {
-                    dma_block<P, i>(ktile, L.dma_k, kdst);
-                } else {
-                    if (v_valid >= kKeyTile) dma_block<P, i - P::DPW>(vtile, L.dma_v, vdst);
-                }
-            });
+            constexpr int i = decltype(dc)::value;
+            static_assert(2 * P::DPW <= S::DT, "a PV MFMA for every DMA block");
+            if constexpr (i < P::DPW) {
+                dma_block<P, i>(ktile, L.dma_k, kdst);
+            } else if constexpr (i < 2 * P::DPW) {
+                if (v_valid >= kKeyTile) dma_block<P, i - P::DPW>(vtile, L.dma_v, vdst);
+            }
         }
     };
     auto dma_partial = [&] {
@@ -741,39 +733,28 @@ __device__ __forceinline__ void overlap_body(FwdArgs& a, uint8_t* lds) {
     if constexpr (SPLIT) {
         if (row_ok) {
             const int64_t prow = (int64_t)split * a.rows_per_head * a.num_kv_heads + row_off / (D * 2);
-            if constexpr (D == 256) {
-                // fp16 partials of O / l, before the v_scale factor (the merge
-                // applies it): a weighted mean of e4m3 V codes, |O / l| <= 448
-                // whatever v_scale is, so fp16 keeps its relative precision;
-                // half the bytes of fp32 for this kernel to write and the merge
-                // to read
-                const float inv_l = sm.l > 0.f ? 1.f / sm.l : 0.f;
-                _Float16* const po = (_Float16*)a.part_o + prow * D;
+            // fp16 partials of O / l, before the v_scale factor (the merge
+            // applies it): a weighted mean of e4m3 V codes, |O / l| <= 448
+            // whatever v_scale is, so fp16 keeps its relative precision;
+            // half the bytes of fp32 for this kernel to write and the merge
+            // to read
+            const float inv_l = sm.l > 0.f ? 1.f / sm.l : 0.f;
+            _Float16* const po = (_Float16*)a.part_o + prow * D;
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
+            for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                    for (int r4 = 0; r4 < 4; ++r4) {
-                        const int d = 32 * dt + 8 * r4 + 4 * h;
-                        uint32_t w[2];
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    const int d = 32 * dt + 8 * r4 + 4 * h;
+                    uint32_t w[2];
 #pragma unroll
-                        for (int i = 0; i < 2; ++i) {
-                            const _Float16 x0 = (_Float16)(o[dt][4 * r4 + 2 * i] * inv_l);
-                            const _Float16 x1 = (_Float16)(o[dt][4 * r4 + 2 * i + 1] * inv_l);
-                            w[i] = (uint32_t)__builtin_bit_cast(uint16_t, x0) |
-                                   ((uint32_t)__builtin_bit_cast(uint16_t, x1) << 16);
-                        }
-                        *(v2i*)(po + d) = v2i{(int)w[0], (int)w[1]};
+                    for (int i = 0; i < 2; ++i) {
+                        const _Float16 x0 = (_Float16)(o[dt][4 * r4 + 2 * i] * inv_l);
+                        const _Float16 x1 = (_Float16)(o[dt][4 * r4 + 2 * i + 1] * inv_l);
+                        w[i] = (uint32_t)__builtin_bit_cast(uint16_t, x0) |
+                               ((uint32_t)__builtin_bit_cast(uint16_t, x1) << 16);
                     }
-            } else {
-                float* const po = a.part_o + prow * D;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                    for (int r4 = 0; r4 < 4; ++r4)
-                        *(v4f*)(po + 32 * dt + 8 * r4 + 4 * h) =
-                            v4f{o[dt][4 * r4] * scale, o[dt][4 * r4 + 1] * scale, o[dt][4 * r4 + 2] * scale,
-                                o[dt][4 * r4 + 3] * scale};
-            }
+                    *(v2i*)(po + d) = v2i{(int)w[0], (int)w[1]};
+                }
             if (h == 0) {
                 a.part_lse[prow] = lse;
                 if (a.part_m) a.part_m[prow] = sm.m;
@@ -817,15 +798,13 @@ __global__ void __launch_bounds__(threads(8), 1) history_fwd_overlap(FwdArgs a) 
     overlap_body<D, FAST, LSE, SPLIT, 8>(a, lds);
 }
 
-// Any head dim and workgroup size.  The LDS (lds_bytes(D)) is dynamic so that
-// the compiler does not see that it leaves a CU one workgroup: it then keeps
-// to 256 VGPRs a wave.  With the four waves of a static 128 KB workgroup it
-// took 368 registers, the accumulators in AGPRs, and copied the scores out of
-// them (head_dim 256, 64 row tiles x 2 ranges of 16 key tiles: 46.4 us against
-// 34; workgroups of 256 rows 44.6).  head_dim 128 and 64 run here rather than
-// on the tile kernel because a wave's softmax issues under its own PV MFMAs:
-// 64 x 8 heads at head_dim 128, 2048 x 30011, 1218 -> 1165 us a call.
-template <int D, bool FAST, bool LSE, bool SPLIT, int WAVES>
+// Four waves, 128 rows.  The LDS (lds_bytes(D)) is dynamic so that the
+// compiler does not see that it leaves a CU one workgroup: it then keeps to
+// 256 VGPRs a wave.  With the four waves of a static 128 KB workgroup it took
+// 368 registers, the accumulators in AGPRs, and copied the scores out of them
+// (head_dim 256, 64 row tiles x 2 ranges of 16 key tiles: 46.4 us against 34;
+// workgroups of 256 rows 44.6).
+template <int D, bool FAST, bool LSE, bool SPLIT, int WAVES = 4>
 __global__ void __launch_bounds__(threads(WAVES), 8 / WAVES) history_fwd_overlap_waves(FwdArgs a) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t dynamic_lds[];
     overlap_body<D, FAST, LSE, SPLIT, WAVES>(a, dynamic_lds);
@@ -851,7 +830,7 @@ constexpr int lds_bytes(int d) { return 2 * kStages * kKeyTile * d; }
 // memory instead of three (2-split 16-rank workload: 0.1761 against 0.1792
 // ms per call; 8-split 4-rank BF16 workload: 0.0124 against 0.0137 ms);
 // NS == 0: any count.
-constexpr int kMergeThreads = 1024;
+constexpr int kMergeThreads = 1024;  // at most: 32 rows of head_dim 256
 template <int NS>
 __global__ void __launch_bounds__(kMergeThreads) merge_splits_kernel(const float* part_o, int part_f16, float part_scale,
                                                            const float* part_lse, int splits, int64_t rows, int d_vec8, uint8_t* out,
@@ -859,7 +838,7 @@ __global__ void __launch_bounds__(kMergeThreads) merge_splits_kernel(const float
                                                            const float* part_m, int32_t* guard_plan, GuardShape g,
                                                            float lse_bias, const float* guard_thr) {
     __shared__ int listed[kGuardMaxHeads];
-    const int64_t idx = (int64_t)blockIdx.x * kMergeThreads + threadIdx.x;
+    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool real = idx < rows * d_vec8;
     if (!guard_plan && !real) return;
     const int64_t row = real ? idx / d_vec8 : rows - 1;

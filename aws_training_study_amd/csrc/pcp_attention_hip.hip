@@ -155,9 +155,18 @@ inline FwdArgs history_args(const pcpa_params* p, const void* q, const void* kv_
     return a;
 }
 
-// The tile kernel instantiation (BF16 MFMAs) for a head dim and cache dtype.
+// The tile kernel instantiation for a head dim, cache dtype and MFMA precision
+// (e4m3 MFMAs below head_dim 256: on the overlap kernel with the tile kernel's
+// running-max rule, head_dim 64 took 602 us against 399 at 24 x 8 heads, 2048
+// x 40960, its two PV MFMAs a tile leaving little to issue the softmax under;
+// head_dim 128 was 4% ahead over 469 key tiles but 4-10% behind over 32-64,
+// and the runtime length is on the GPU).
 template <bool SPLIT>
-inline const void* tile_kernel_for(int head_dim, bool store8) {
+inline const void* tile_kernel_for(int head_dim, bool store8, bool fp8) {
+    if (fp8)
+        return head_dim == 64    ? (const void*)history_fwd_kernel<64, true, true, false, SPLIT>
+               : head_dim == 128 ? (const void*)history_fwd_kernel<128, true, true, false, SPLIT>
+                                 : nullptr;
     switch (head_dim * 2 + (store8 ? 1 : 0)) {
         case 64 * 2 + 1: return (const void*)history_fwd_kernel<64, true, false, false, SPLIT>;
         case 128 * 2 + 1: return (const void*)history_fwd_kernel<128, true, false, false, SPLIT>;
@@ -171,41 +180,25 @@ inline const void* tile_kernel_for(int head_dim, bool store8) {
 
 constexpr int kComputeUnits = 256;  // MI355X
 
-// The e4m3-MFMA kernel: head_dim 256 with either exp2, head_dim 64 and 128
-// with the exact one; per-row values (aux: log-sum-exp, guard rows) or split
-// partials.
-template <int WAVES>
-inline const void* overlap_waves_for(int head_dim, bool fast, bool aux, bool split) {
+// The overlap kernel (e4m3 MFMAs at head_dim 256): either exp2, per-row values
+// (aux: log-sum-exp, guard rows) or split partials, four waves (always with
+// the per-row values: one instantiation) or eight.
+inline const void* overlap_kernel_for(bool fast, bool aux, bool split, int waves) {
     using namespace ovl;
-    switch (head_dim) {
-        case 64:
-            return split ? (const void*)history_fwd_overlap_waves<64, false, false, true, WAVES>
-                         : (const void*)history_fwd_overlap_waves<64, false, true, false, WAVES>;
-        case 128:
-            return split ? (const void*)history_fwd_overlap_waves<128, false, false, true, WAVES>
-                         : (const void*)history_fwd_overlap_waves<128, false, true, false, WAVES>;
-        default: break;
-    }
-    if constexpr (WAVES == 4) {
-        if (head_dim != 256) return nullptr;
+    if (waves == 4) {
         if (split)
-            return fast ? (const void*)history_fwd_overlap_waves<256, true, false, true, 4>
-                        : (const void*)history_fwd_overlap_waves<256, false, false, true, 4>;
-        return fast ? (const void*)history_fwd_overlap_waves<256, true, true, false, 4>
-                    : (const void*)history_fwd_overlap_waves<256, false, true, false, 4>;
+            return fast ? (const void*)history_fwd_overlap_waves<256, true, false, true>
+                        : (const void*)history_fwd_overlap_waves<256, false, false, true>;
+        return fast ? (const void*)history_fwd_overlap_waves<256, true, true, false>
+                    : (const void*)history_fwd_overlap_waves<256, false, true, false>;
     }
-    return nullptr;
-}
-inline const void* overlap_kernel_for(int head_dim, bool fast, bool aux, bool split, int waves) {
-    if (waves == 4) return overlap_waves_for<4>(head_dim, fast, aux, split);
-    if (head_dim != 256) return overlap_waves_for<8>(head_dim, fast, aux, split);
     if (split)
-        return fast ? (const void*)ovl::history_fwd_overlap<256, true, false, true>
-                    : (const void*)ovl::history_fwd_overlap<256, false, false, true>;
-    return fast ? (aux ? (const void*)ovl::history_fwd_overlap<256, true, true>
-                       : (const void*)ovl::history_fwd_overlap<256, true, false>)
-                : (aux ? (const void*)ovl::history_fwd_overlap<256, false, true>
-                       : (const void*)ovl::history_fwd_overlap<256, false, false>);
+        return fast ? (const void*)history_fwd_overlap<256, true, false, true>
+                    : (const void*)history_fwd_overlap<256, false, false, true>;
+    return fast ? (aux ? (const void*)history_fwd_overlap<256, true, true>
+                       : (const void*)history_fwd_overlap<256, true, false>)
+                : (aux ? (const void*)history_fwd_overlap<256, false, true>
+                       : (const void*)history_fwd_overlap<256, false, false>);
 }
 
 // Device memory of the guard scratch (see guard_scratch below), held for
@@ -285,11 +278,11 @@ inline int32_t history_launch(const pcpa_params* p, int splits, const void* q, c
     // e4m3 MFMAs: a workgroup of eight waves takes 256 rows and a CU; where
     // workgroups of 128 rows (four waves) still find a CU each they finish
     // sooner, a wave then having its SIMD to itself (4 ranks x 256 tokens over
-    // 2048 keys: 96.4 -> 84.5 us a call), and beyond that they take turns
-    // (64 x 8 heads at head_dim 128, 2048 x 30011: 1240 against 1165 us)
-    const bool narrow = fp8 && (int64_t)a.row_tiles * p->num_kv_heads * splits <= kComputeUnits;
+    // 2048 keys: 96.4 -> 84.5 us a call)
+    const bool overlap = fp8 && p->head_dim == 256;
+    const bool narrow = overlap && (int64_t)a.row_tiles * p->num_kv_heads * splits <= kComputeUnits;
     const int waves = narrow ? 4 : 8;
-    const int rows_per_group = fp8 ? ovl::rows_per_group(waves) : kRowsPerGroup;
+    const int rows_per_group = overlap ? ovl::rows_per_group(waves) : kRowsPerGroup;
     a.row_tiles = (a.rows_per_head + rows_per_group - 1) / rows_per_group;
     if (splits == 1) {
         // a guarded pass lists its rows below the threshold itself
@@ -303,18 +296,18 @@ inline int32_t history_launch(const pcpa_params* p, int splits, const void* q, c
         a.part_m = guard ? (float*)(ws + w.part_m) : nullptr;
     }
     const void* fn;
-    if (fp8)
+    if (overlap)
         // one pass: the log-sum-exp instantiation also lists the guard's rows
-        fn = overlap_kernel_for(p->head_dim, fast, lse || guard, splits > 1, waves);
+        fn = overlap_kernel_for(fast, lse || guard, splits > 1, waves);
     else if (splits == 1)
-        fn = tile_kernel_for<false>(p->head_dim, store8);
+        fn = tile_kernel_for<false>(p->head_dim, store8, fp8);
     else
-        fn = tile_kernel_for<true>(p->head_dim, store8);
+        fn = tile_kernel_for<true>(p->head_dim, store8, fp8);
     if (!fn) return PCPA_ERR_UNSUPPORTED;
     void* args[] = {&a};
     const int items = a.row_tiles * p->num_kv_heads * splits;
-    const int threads = fp8 ? ovl::threads(waves) : tile_threads(p->head_dim, false);
-    const size_t lds = fp8 && (narrow || p->head_dim != 256) ? ovl::lds_bytes(p->head_dim) : 0;
+    const int threads = overlap ? ovl::threads(waves) : tile_threads(p->head_dim, fp8);
+    const size_t lds = narrow ? ovl::lds_bytes(p->head_dim) : 0;
     if (hipLaunchKernel(fn, dim3(8 * ((items + 7) / 8)), dim3(threads), args, lds, stream) != hipSuccess)
         return PCPA_ERR_LAUNCH;
     GuardShape g{};
@@ -334,8 +327,9 @@ inline int32_t history_launch(const pcpa_params* p, int splits, const void* q, c
         auto merge = splits == 2 ? merge_splits_kernel<2> : splits == 3 ? merge_splits_kernel<3>
                    : splits == 4 ? merge_splits_kernel<4> : splits == 8 ? merge_splits_kernel<8>
                    : merge_splits_kernel<0>;
-        hipLaunchKernelGGL(merge, dim3((unsigned)((threads + kMergeThreads - 1) / kMergeThreads)),
-                           dim3(kMergeThreads), 0, stream,
+        // 32 rows a workgroup share one list atomic per KV head
+        const int per_group = guard ? 32 * d_vec8 : 256;
+        hipLaunchKernelGGL(merge, dim3((unsigned)((threads + per_group - 1) / per_group)), dim3(per_group), 0, stream,
                            (const float*)a.part_o, a.part_f16, a.part_f16 ? p->v_scale : 1.f,
                            (const float*)a.part_lse, splits, g.rows_total, d_vec8,
                            (uint8_t*)out, lse, (const float*)a.part_m, plan, g, fp8 && p->head_dim == 256 && fast ? kFastLseBias : 0.f,

@@ -89,15 +89,16 @@ __device__ __forceinline__ void stage_tile_async(const FwdArgs& a, const TileCur
                                                  const LaneMap<S>& L) {
     const uint8_t* const kt = a.kv + c.k_off + (int64_t)c.base * S::ROW;
     const uint8_t* const vt = kt + (int64_t)a.num_kv_heads * a.head_stride;
-    // (the opaque base keeps each block's address computation next to its
-    // load: all of them ahead of the first load delay the whole burst)
     uint32_t dst = lds_address(lk) + wave * 1024;
 #pragma unroll
     for (int i = 0; i < S::DMA_PER_WAVE; ++i) {
         const int delta = S::dma_key_delta(i) * S::ROW;
-        asm volatile("" : "+s"(dst));
+        // bf16: the opaque base keeps each block's address computation next
+        // to its load (all of them ahead of the first load delay the burst of
+        // eight); the e4m3 tiles' two to four blocks are better without
+        if constexpr (!S::F8) asm volatile("" : "+s"(dst));
         dma_sbase<0>(kt + delta, L.dma_off, dst + S::WAVES * i * 1024);
-        asm volatile("" : "+s"(dst));
+        if constexpr (!S::F8) asm volatile("" : "+s"(dst));
         dma_sbase<0>(vt + delta, L.dma_off_v, dst + S::TILE + S::WAVES * i * 1024);
     }
 }
@@ -432,48 +433,41 @@ __device__ __forceinline__ void compute_tile(const uint8_t* lds, uint32_t rt_off
     }
 }
 
-// Wait for the step's tiles `cur` (in BUF; TILES of them, the second possibly
-// past the last), start the prefetch of `nxt` into the other buffer, then
-// compute this wave's tile of `cur`.
+// Wait for tile `cur` (in BUF; TILES 2: and `cur2`, possibly past the last),
+// start the prefetch of `nxt` (and `nxt2`) into the other buffer, then compute
+// this wave's tile.
 // PAIR: BUF is 0 and rbuf the buffer of `cur`, so that the walk has one loop
 // body (two bodies made the register allocator keep copies of O^T across
 // them and spill).
 template <class S, int BUF, bool CAUSAL>
-__device__ __forceinline__ void tile_step(const FwdArgs& a, const TileCursor (&cur)[S::TILES],
-                                          const TileCursor (&nxt)[S::TILES], uint8_t* lds, int wave, int tid, int h,
-                                          const LaneMap<S>& L, const QOperand<S> (&qop)[S::QK],
+__device__ __forceinline__ void tile_step(const FwdArgs& a, const TileCursor& cur, const TileCursor& cur2,
+                                          const TileCursor& nxt, const TileCursor& nxt2, uint8_t* lds, int wave,
+                                          int tid, int h, const LaneMap<S>& L, const QOperand<S> (&qop)[S::QK],
                                           float cscale, SoftmaxState<S>& st, int row_limit, int kh, int rbuf) {
+    constexpr bool TWO = S::TILES == 2;
+    const int valid = min(kKeyTile, cur.n - cur.base);
+    const int valid2 = TWO ? min(kKeyTile, cur2.n - cur2.base) : 0;  // 0 past the last tile
     const uint32_t rt_off = S::PAIR ? rbuf * S::BUFFER : 0;
     uint8_t* const buf = lds + BUF * S::BUFFER + rt_off;
-    int valid[S::TILES];
-    bool partial = false;
-#pragma unroll
-    for (int i = 0; i < S::TILES; ++i) {
-        valid[i] = min(kKeyTile, cur[i].n - cur[i].base);  // 0 past the last tile
-        partial |= valid[i] < kKeyTile && (S::TILES == 1 || valid[i] > 0);
-    }
     wait_vmem();      // this wave's loads of the current tiles have landed
     __syncthreads();  // ... and every wave's; the other buffer is free
-#pragma unroll
-    for (int i = 0; i < S::TILES; ++i)
-        if (nxt[i].e < a.num_entries) {
-            uint8_t* const other = lds + (S::PAIR ? rt_off ^ S::BUFFER : (BUF ^ 1) * S::BUFFER);
-            stage_tile_async<S>(a, nxt[i], other + i * 2 * S::TILE, wave, L);
-        }
-    if (partial) {
-#pragma unroll
-        for (int i = 0; i < S::TILES; ++i)
-            if (S::TILES == 1 || valid[i] > 0) zero_masked_v<S>(buf + i * 2 * S::TILE + S::TILE, valid[i], tid);
+    if (nxt.e < a.num_entries) {
+        uint8_t* const other = lds + (S::PAIR ? rt_off ^ S::BUFFER : (BUF ^ 1) * S::BUFFER);
+        stage_tile_async<S>(a, nxt, other, wave, L);
+        if (TWO && nxt2.e < a.num_entries) stage_tile_async<S>(a, nxt2, other + 2 * S::TILE, wave, L);
+    }
+    if (valid < kKeyTile || (TWO && valid2 > 0 && valid2 < kKeyTile)) {
+        if (!TWO || valid < kKeyTile) zero_masked_v<S>(buf + S::TILE, valid, tid);
+        if (TWO && valid2 > 0 && valid2 < kKeyTile) zero_masked_v<S>(buf + 3 * S::TILE, valid2, tid);
         __syncthreads();
     }
-    if constexpr (S::TILES == 2) {
-        const int v = kh ? valid[1] : valid[0];
+    if constexpr (TWO) {
+        const int v = kh ? valid2 : valid;
         if (v > 0) compute_tile<S, BUF, CAUSAL>(lds, rt_off + kh * 2 * S::TILE, v, qop, cscale, L, h, st);
     } else {
         const int first_key = S::PAIR ? 32 * kh : 0;
-        compute_tile<S, BUF, CAUSAL>(lds, rt_off,
-                                     (CAUSAL ? min(valid[0], row_limit - cur[0].base) : valid[0]) - first_key, qop,
-                                     cscale, L, h, st);
+        compute_tile<S, BUF, CAUSAL>(lds, rt_off, (CAUSAL ? min(valid, row_limit - cur.base) : valid) - first_key,
+                                     qop, cscale, L, h, st);
     }
 }
 
@@ -757,40 +751,32 @@ __global__ void __launch_bounds__((TileShape<D, STORE8, FP8>::THREADS), (TileSha
         }
     };
 
-    // the next step's tiles after `last`
-    auto next_step = [&](TileCursor last, TileCursor (&t)[S::TILES]) {
-#pragma unroll
-        for (int i = 0; i < S::TILES; ++i) t[i] = last = advance(last);
-    };
-    TileCursor cur[S::TILES], nxt[S::TILES];
-    if (FIXUP && sparse) {
-        cur[0] = range_first;
-        if constexpr (S::TILES == 2) cur[1] = advance(cur[0]);
-    } else {
-        next_step(TileCursor{entry_begin - 1, 0, 0, 0}, cur);
-    }
-#pragma unroll
-    for (int i = 0; i < S::TILES; ++i)
-        if (cur[i].e < a.num_entries) stage_tile_async<S>(a, cur[i], lds + i * 2 * S::TILE, wave, L);
-    auto take_next = [&] {
-#pragma unroll
-        for (int i = 0; i < S::TILES; ++i) cur[i] = nxt[i];
-    };
+    constexpr bool TWO = S::TILES == 2;
+    TileCursor cur, cur2{};
+    if (FIXUP && sparse)
+        cur = range_first;
+    else
+        cur = advance(TileCursor{entry_begin - 1, 0, 0, 0});
+    if constexpr (TWO) cur2 = advance(cur);
+    if (cur.e < a.num_entries) stage_tile_async<S>(a, cur, lds, wave, L);
+    if (TWO && cur2.e < a.num_entries) stage_tile_async<S>(a, cur2, lds + 2 * S::TILE, wave, L);
     if constexpr (S::PAIR) {
-        for (int rbuf = 0; cur[0].e < a.num_entries; rbuf ^= 1) {
-            next_step(cur[S::TILES - 1], nxt);
-            tile_step<S, 0, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, kh, rbuf);
-            take_next();
+        for (int rbuf = 0; cur.e < a.num_entries; rbuf ^= 1) {
+            const TileCursor nxt = advance(TWO ? cur2 : cur);
+            const TileCursor nxt2 = TWO ? advance(nxt) : TileCursor{};
+            tile_step<S, 0, CAUSAL>(a, cur, cur2, nxt, nxt2, lds, wave, tid, h, L, qop, cscale, st, row_limit, kh, rbuf);
+            cur = nxt;
+            cur2 = nxt2;
         }
     } else {
-        while (cur[0].e < a.num_entries) {
-            next_step(cur[0], nxt);
-            tile_step<S, 0, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, kh, 0);
-            take_next();
-            if (cur[0].e >= a.num_entries) break;
-            next_step(cur[0], nxt);
-            tile_step<S, 1, CAUSAL>(a, cur, nxt, lds, wave, tid, h, L, qop, cscale, st, row_limit, kh, 0);
-            take_next();
+        while (cur.e < a.num_entries) {
+            TileCursor nxt = advance(cur);
+            tile_step<S, 0, CAUSAL>(a, cur, cur2, nxt, cur2, lds, wave, tid, h, L, qop, cscale, st, row_limit, 0, 0);
+            cur = nxt;
+            if (cur.e >= a.num_entries) break;
+            nxt = advance(cur);
+            tile_step<S, 1, CAUSAL>(a, cur, cur2, nxt, cur2, lds, wave, tid, h, L, qop, cscale, st, row_limit, 0, 0);
+            cur = nxt;
         }
     }
 
