@@ -176,6 +176,33 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+_fast_calls = None
+
+
+def fast_calls():
+    """The extension module of the per-call host path (``csrc/fast_calls.cpp``)."""
+    global _fast_calls
+    if _fast_calls is None:
+        import importlib.util
+
+        import torch  # noqa: F401  (its libraries hold the extension's symbols)
+
+        path = Path(__file__).resolve().parent / "_lib" / "_pcpa_fast_calls.so"
+        if not path.exists():
+            raise RuntimeError(f"extension {path} is missing; build it with "
+                               "`python -c 'import __graft_entry__ as g; g.build()'`")
+        spec = importlib.util.spec_from_file_location("_pcpa_fast_calls", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _fast_calls = module
+    return _fast_calls
+
+
+def function_address(fn) -> int:
+    """Address of a function of the loaded library."""
+    return ctypes.cast(fn, ctypes.c_void_p).value
+
+
 def status_string(status: int) -> str:
     return load_library().pcpa_status_string(status).decode()
 

@@ -3,8 +3,10 @@
 ``python -m aws_training_study_amd.build_native`` compiles
 ``csrc/pcp_attention_hip.hip`` (which includes the kernel headers in
 ``csrc/``) into ``_lib/libpcp_attention_hip.so``.  hipcc cross-compiles for
-gfx950 without a GPU present.  Then gcc builds ``csrc/abi_example.c``, a
-plain C caller of the library, into ``_lib/abi_example``.
+gfx950 without a GPU present.  Then g++ builds ``csrc/fast_calls.cpp``, the
+Python entry points' per-call host path, into ``_lib/_pcpa_fast_calls.so`` and
+gcc ``csrc/abi_example.c``, a plain C caller of the library, into
+``_lib/abi_example``.
 """
 
 from __future__ import annotations
@@ -20,6 +22,8 @@ REPO_ROOT = PACKAGE_DIR.parent
 SOURCES = [PACKAGE_DIR / "csrc" / "pcp_attention_hip.hip"]
 INCLUDE_DIR = REPO_ROOT / "include"
 OUTPUT = PACKAGE_DIR / "_lib" / "libpcp_attention_hip.so"
+FAST_CALLS_SOURCE = PACKAGE_DIR / "csrc" / "fast_calls.cpp"
+FAST_CALLS = PACKAGE_DIR / "_lib" / "_pcpa_fast_calls.so"
 EXAMPLE_SOURCE = PACKAGE_DIR / "csrc" / "abi_example.c"
 EXAMPLE = PACKAGE_DIR / "_lib" / "abi_example"
 OFFLOAD_ARCH = "gfx950"
@@ -85,6 +89,47 @@ def example_command(output: Path = EXAMPLE) -> list[str]:
     ]
 
 
+def fast_calls_command(output: Path = FAST_CALLS) -> list[str]:
+    """g++ line of the CPython extension over torch's C++ tensors (linked to
+    the libraries that ``import torch`` has loaded by then)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    return [
+        "g++",
+        "-O2",
+        "-std=c++17",
+        "-shared",
+        "-fPIC",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f"-I{INCLUDE_DIR}",
+        f"-I{sysconfig.get_paths()['include']}",
+        *[f"-I{path}" for path in cpp_extension.include_paths()],
+        os.fspath(FAST_CALLS_SOURCE),
+        *[f"-L{path}" for path in cpp_extension.library_paths()],
+        "-ltorch_python",
+        "-ltorch_cpu",
+        "-lc10",
+        "-o",
+        os.fspath(output),
+    ]
+
+
+def build_fast_calls(verbose: bool = False) -> Path:
+    """Compile the per-call host path of the Python entry points."""
+    tmp = FAST_CALLS.with_suffix(".so.tmp")
+    cmd = fast_calls_command(tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"g++ failed ({result.returncode}):\n{result.stderr}")
+    os.replace(tmp, FAST_CALLS)
+    return FAST_CALLS
+
+
 def build_example(verbose: bool = False) -> Path:
     """Compile the C caller against the built library."""
     cmd = example_command()
@@ -111,6 +156,7 @@ def build(verbose: bool = False) -> Path:
     if verbose and stderr.strip():
         print(stderr, file=sys.stderr)
     os.replace(tmp, OUTPUT)
+    build_fast_calls(verbose)
     build_example(verbose)
     return OUTPUT
 

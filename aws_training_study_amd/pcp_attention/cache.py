@@ -79,9 +79,18 @@ class KVCacheWriter:
             softmax_scale=cfg.softmax_scale,
             flags=0,
         )
+        self._fast = None  # the native call, made by the first one
 
     def __call__(self, k, v, kv_pages, block_table, *, first_pos: int = 0, k_scale: float = 1.0,
                  v_scale: float = 1.0, page_valid_len: Optional[object] = None) -> None:
+        if self._fast is None:
+            params = self._native.PcpaParams(num_pages=self.config.num_pages, k_scale=1.0, v_scale=1.0, **self._static)
+            self._fast = self._native.fast_calls().make(
+                "write", bytes(params), self.config.kv_dtype == "fp8_e4m3fn", self.config.interleave_size,
+                self._native.function_address(self._lib.pcpa_kv_cache_write))
+        if self._fast(k, v, kv_pages, block_table, first_pos, k_scale, v_scale, page_valid_len):
+            return
+        # not the common form, or an error
         import torch
 
         cfg = self.config
@@ -178,6 +187,7 @@ class PageAllocator:
             max_local_blocks=self.config.max_local_blocks, num_pages=self.num_pages, q_dtype=_native.DTYPE_BF16,
             kv_dtype=_KV_DTYPE_CODES[self.config.kv_dtype], out_dtype=_native.DTYPE_BF16,
             softmax_scale=self.config.softmax_scale, k_scale=1.0, v_scale=1.0, flags=0)
+        self._fast = None  # the native call, made by the first allocation
 
     def empty_table(self, dtype=None):
         """A block table with no page assigned (every entry -1)."""
@@ -189,6 +199,13 @@ class PageAllocator:
 
     def allocate(self, first_pos: int, num_tokens: int, block_table) -> None:
         """Assign pages to the blocks that positions [first_pos, first_pos + num_tokens) reach (asynchronous)."""
+        if self._fast is None:
+            self._fast = self._native.fast_calls().make(
+                "alloc", bytes(self._params), False, self.config.interleave_size,
+                self._native.function_address(self._lib.pcpa_page_alloc))
+        if self._fast(first_pos, num_tokens, block_table, self.free_pages, self.free_count):
+            return
+        # not the common form, or an error
         import torch
 
         cfg = self.config

@@ -82,8 +82,17 @@ class CurrentAttentionKernel:
         status = self._lib.pcpa_check_params(ctypes.byref(self._launch_params))
         if status != _native.PCPA_OK:
             raise ValueError(f"configuration rejected by the HIP kernel: {_native.status_string(status)}")
+        self._fast = None  # the native call, made by the first one
 
     def __call__(self, q, kv_current, hist_out=None, hist_lse=None, *, out=None, return_lse: bool = False):
+        if self._fast is None:
+            self._fast = self._native.fast_calls().make(
+                "current", bytes(self._launch_params), False, self.config.interleave_size,
+                self._native.function_address(self._lib.pcpa_current_attention))
+        result = self._fast(q, kv_current, hist_out, hist_lse, out, return_lse)
+        if result is not None:
+            return result
+        # not the common form, or an error
         import torch
 
         cfg = self.config

@@ -151,6 +151,7 @@ class HistoryAttentionKernel:
         self._ws_sizes = {}
         self._split_ws = {}
         self._local_pools = {}
+        self._plans = {}  # (precision, exp2, splits) -> the native call of that form
         self._q_shape = (cfg.pcp_size, cfg.num_q_heads, cfg.local_q_len, cfg.head_dim)
         self._table_shape = (cfg.pcp_size, cfg.max_local_blocks)
         self._modes = {p: (self.uses_bf16_mfma(p), self.guarded(p)) for p in PRECISIONS}
@@ -216,6 +217,17 @@ class HistoryAttentionKernel:
         splits="auto",
         workspace=None,
     ):
+        if page_valid_len is not None and block_valid_mask is None and workspace is None:
+            # the common form of the call, checked and launched natively;
+            # None: not that form (or an error), which the rest of this
+            # function sees to
+            plan = self._plans.get((precision, exp2, splits))
+            if plan is None:
+                plan = self._plan(precision, exp2, splits, page_valid_len)
+            if plan is not None:
+                result = plan(q, kv_pages, block_table, page_valid_len, k_scale, v_scale, out, return_lse)
+                if result is not None:
+                    return result
         import torch
 
         cfg = self.config
@@ -323,6 +335,38 @@ class HistoryAttentionKernel:
         if status:
             self._native.check(status)
         return (out, lse) if return_lse else out
+
+    def _plan(self, precision, exp2, splits, page_valid_len):
+        """The native call of this form on the lengths' GPU, kept; ``None`` for
+        lengths that are not on a GPU and for options the general path refuses."""
+        import weakref
+
+        if (precision not in PRECISIONS or exp2 not in EXP2_MODES or not (splits == "auto" or type(splits) is int)
+                or not getattr(page_valid_len, "is_cuda", False)):
+            return None
+        device = page_valid_len.device
+        bf16_mfma, guard = self._modes[precision]
+        n_split = self.split_count(device, bf16_mfma) if splits == "auto" else splits
+        params = self._params(self.config.num_pages, 1.0, 1.0)
+        if bf16_mfma:
+            params.flags |= self._native.FLAG_BF16_MFMA
+        if exp2 == "exact":
+            params.flags |= self._native.FLAG_EXACT_EXP2
+        if guard:
+            params.flags |= self._native.FLAG_PRECISION_GUARD
+        elif not bf16_mfma:
+            params.flags |= self._native.FLAG_E4M3_UNGUARDED
+        split = n_split > 1 or guard
+        fn = self._lib.pcpa_history_attention_split if split else self._lib.pcpa_history_attention_lse
+        me = weakref.ref(self)  # (the plan is ours: no cycle that keeps workspaces until a collection)
+        plan = self._native.fast_calls().make_history(
+            bytes(params), self.config.kv_dtype == "fp8_e4m3fn", self._native.function_address(fn), device.index,
+            n_split, self.workspace_bytes(n_split, precision) if split else -1,
+            lambda size, stream: me()._workspace(size, device, stream))
+        if len(self._plans) >= 64:
+            self._plans.clear()
+        self._plans[(precision, exp2, splits)] = plan
+        return plan
 
     def pool_from_local_caches(self, local_kv, device=None):
         """(pool, identity block table) of the reference's per-rank caches.
@@ -476,6 +520,8 @@ class HistoryAttentionKernel:
                 self._split_ws.clear()
             ws = torch.empty(max(size, 16), dtype=torch.uint8, device=device)
             self._split_ws[key] = ws
+            for plan in self._plans.values():
+                plan.forget()  # workspaces dropped here are dropped there too
         return ws
 
 

@@ -1,0 +1,114 @@
+"""The native per-call path of the Python entry points (csrc/fast_calls.cpp).
+
+It takes the common form of the arguments and leaves every other form to the
+general path: same results, same conversions, same errors.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from aws_training_study_amd.pcp_attention import (
+    KVCacheWriter,
+    PageAllocator,
+    PCPAttentionConfig,
+    append_history,
+    build_page_pool,
+    make_history_attention_kernel,
+)
+from aws_training_study_amd.pcp_attention.current import CurrentAttentionKernel
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(device, kv_dtype="fp8_e4m3fn"):
+    cfg = PCPAttentionConfig(pcp_size=2, current_len=128, max_history_len=512, actual_history_len=512, block_size=128,
+                             interleave_size=64, num_q_heads=4, num_kv_heads=2, head_dim=64, backend="hip",
+                             kv_dtype=kv_dtype).validate()
+    gen = torch.Generator(device=device).manual_seed(1)
+
+    def normal(*shape):
+        return torch.randn(shape, generator=gen, device=device, dtype=torch.bfloat16)
+
+    table = torch.arange(cfg.num_pages, device=device, dtype=torch.int32).flip(0).reshape(2, -1).contiguous()
+    pool, k_scale, v_scale, valid = build_page_pool(cfg, normal(2, 500, 64), normal(2, 500, 64), table)
+    return cfg, normal(2, 4, 64, 64), pool, table, valid, k_scale, v_scale
+
+
+@pytest.mark.parametrize("kv_dtype,precision,splits", [("fp8_e4m3fn", "auto", "auto"), ("fp8_e4m3fn", "fp8", 1),
+                                                       ("fp8_e4m3fn", "bf16", 3), ("bfloat16", "auto", "auto")])
+def test_history_common_form_equals_the_general_path(kv_dtype, precision, splits, cuda_device):
+    cfg, q, pool, table, valid, k_scale, v_scale = _case(cuda_device, kv_dtype)
+    kernel = make_history_attention_kernel(cfg)
+    kw = dict(page_valid_len=valid, k_scale=k_scale, v_scale=v_scale, precision=precision, splits=splits)
+    # an int64 copy of the lengths: the general path
+    first = kernel(q, pool, table, return_lse=True, **dict(kw, page_valid_len=valid.long()))
+    other = torch.empty_like(q)
+    for _ in range(2):
+        out, lse = kernel(q, pool, table, return_lse=True, **kw)
+        assert torch.equal(out, first[0]) and torch.equal(lse, first[1])
+        assert kernel(q, pool, table, out=other, **kw) is not None and torch.equal(other, first[0])
+        assert torch.equal(kernel(q, pool, table.long(), **kw), first[0])
+    # another stream gets a workspace of its own
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        out = kernel(q, pool, table, **kw)
+    side.synchronize()
+    assert torch.equal(out, first[0])
+    # forms left to the general path
+    assert torch.equal(kernel(q, pool, table.cpu(), **kw), first[0])
+    kw_cpu = dict(kw, page_valid_len=valid.cpu().long(), k_scale=torch.tensor(k_scale), splits=splits)
+    assert (kernel(q, pool, table, **kw_cpu).float() - first[0].float()).abs().max() <= 1e-2
+    with pytest.raises(ValueError, match="q must be contiguous bfloat16"):
+        kernel(q.transpose(2, 3), pool, table, **kw)
+    with pytest.raises(ValueError, match="q must be contiguous bfloat16"):
+        kernel(q.float(), pool, table, **kw)
+    with pytest.raises(ValueError, match="GPU tensor"):
+        kernel(q.cpu(), pool, table, **kw)
+    with pytest.raises(ValueError, match="block_table must be"):
+        kernel(q, pool, table[:, :-1].contiguous(), **kw)
+    with pytest.raises(ValueError, match="kv_pages must be contiguous"):
+        kernel(q, pool.view(torch.uint8), table, **kw)
+    with pytest.raises(ValueError, match="out must be contiguous"):
+        kernel(q, pool, table, out=other.float(), **kw)
+    with pytest.raises(ValueError, match="not both"):
+        kernel(q, pool, table, torch.zeros(2, 1, 1, 128), **kw)
+
+
+def test_current_and_cache_calls(cuda_device):
+    cfg, q, _, _, _, _, _ = _case(cuda_device)
+    kv = torch.randn((2, 2, 128, 64), device=cuda_device, dtype=torch.bfloat16)
+    step = CurrentAttentionKernel(cfg)
+    out, lse = step(q, kv, return_lse=True)
+    assert torch.equal(step(q, kv), out)
+    with pytest.raises(ValueError, match="kv_current must be"):
+        step(q, kv[:, :, :64].contiguous())
+    with pytest.raises(ValueError, match="pass both"):
+        step(q, kv, out)
+
+    def fresh():
+        allocator = PageAllocator(cfg, cuda_device)
+        return (allocator, torch.zeros((cfg.num_pages, cfg.page_elements), dtype=torch.float8_e4m3fn,
+                                       device=cuda_device), allocator.empty_table(),
+                torch.zeros((2, cfg.max_local_blocks), dtype=torch.int32, device=cuda_device))
+
+    x = torch.randn((2, 300, 64), device=cuda_device, dtype=torch.bfloat16)
+    writer = KVCacheWriter(cfg)
+    a, b = fresh(), fresh()
+    append_history(writer, a[0], x, x, a[1], a[2], a[3], first_pos=7, k_scale=0.01, v_scale=0.02)
+    # scales that are not Python floats: the general path
+    append_history(writer, b[0], x, x, b[1], b[2], b[3], first_pos=7, k_scale=torch.tensor(0.01),
+                   v_scale=torch.tensor(0.02))
+    for s, t in zip(a[1:], b[1:]):
+        assert torch.equal(s.view(torch.uint8), t.view(torch.uint8))
+    assert int(a[0].free_count) == int(b[0].free_count) < cfg.num_pages
+    with pytest.raises(ValueError, match="v must be a contiguous bfloat16"):
+        writer(x, x[:, :5].contiguous(), a[1], a[2])
+    with pytest.raises(ValueError, match="kv_pages must be"):
+        writer(x, x, a[1].view(torch.uint8), a[2])
+    with pytest.raises(RuntimeError, match="BAD_SHAPE"):
+        writer(x, x, a[1], a[2], first_pos=400)
+    with pytest.raises(RuntimeError, match="BAD_SHAPE"):
+        a[0].allocate(400, 300, a[2])
