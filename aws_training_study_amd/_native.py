@@ -64,7 +64,9 @@ EXPORTED_SYMBOLS = (
     "pcpa_split_workspace_bytes",
     "pcpa_current_attention",
     "pcpa_kv_cache_write",
+    "pcpa_kv_cache_fill",
     "pcpa_absmax_bf16",
+    "pcpa_absmax_pair_bf16",
     "pcpa_block_mask_valid_len",
     "pcpa_page_alloc",
 )
@@ -163,6 +165,12 @@ def load_library() -> ctypes.CDLL:
     ]
     lib.pcpa_absmax_bf16.restype = ctypes.c_int32
     lib.pcpa_absmax_bf16.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
+    lib.pcpa_absmax_pair_bf16.restype = ctypes.c_int32
+    lib.pcpa_absmax_pair_bf16.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+                                          ctypes.c_void_p]
+    lib.pcpa_kv_cache_fill.restype = ctypes.c_int32
+    lib.pcpa_kv_cache_fill.argtypes = [ctypes.POINTER(PcpaParams), ctypes.c_int32, ctypes.c_int32] + [
+        ctypes.c_void_p] * 7
     lib.pcpa_block_mask_valid_len.restype = ctypes.c_int32
     lib.pcpa_block_mask_valid_len.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
                                               ctypes.c_void_p, ctypes.c_void_p]

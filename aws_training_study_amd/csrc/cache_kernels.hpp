@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "paging_kernels.hpp"
 
 // ============================================================================
 // KV-cache producer: per-tensor e4m3 quantisation of K/V and the page write
@@ -58,7 +59,15 @@ struct WriteArgs {
     float k_scale, v_scale;
     float k_rcp, v_rcp;  // RN(1 / scale), for div_rn when fast_div
     int32_t fast_div;    // both scales in [2^-80, 2^126]: div_rn instead of the IEEE division
+    const float* amax;   // optional: max |K| and |V|, which give the scales instead (scale_of)
 };
+
+// The per-tensor e4m3 scale of a tensor whose largest magnitude is `amax`: 1
+// for 0 and NaN.  amax is a bf16 value; its quotient by 448 = 7 * 64 repeats
+// with period 3 in binary and is never near the middle of two floats, so that
+// rounding it once (here) or to double first (on the host) gives the same.
+__device__ __forceinline__ float scale_of(float amax) { return amax > 0.f ? amax / kFp8Max : 1.f; }
+__host__ __device__ __forceinline__ bool div_rn_covers(float scale) { return scale >= 0x1p-80f && scale <= 0x1p126f; }
 
 // x / d rounded to nearest even, as the IEEE division rounds it, from y =
 // RN(1 / d) by Markstein's correction (P. Markstein, IBM J. Res. Develop.
@@ -162,6 +171,13 @@ __global__ void __launch_bounds__(kThreads) kv_write_kernel(WriteArgs a, uint32_
             vf[2 * w] = bf16_bits_to_f32((uint32_t)vin[w] & 0xffffu);
             vf[2 * w + 1] = bf16_bits_to_f32((uint32_t)vin[w] >> 16);
         }
+        if (a.amax) {
+            a.k_scale = scale_of(a.amax[0]);
+            a.v_scale = scale_of(a.amax[1]);
+            a.k_rcp = 1.f / a.k_scale;
+            a.v_rcp = 1.f / a.v_scale;
+            a.fast_div = div_rn_covers(a.k_scale) && div_rn_covers(a.v_scale);
+        }
         // x / scale rounded as torch's (x / scale).to(float8) rounds it
         if (a.fast_div) {
 #pragma unroll
@@ -191,9 +207,68 @@ __global__ void __launch_bounds__(kThreads) kv_write_kernel(WriteArgs a, uint32_
     }
 }
 
+struct FillArgs {
+    const int32_t* block_table;
+    int32_t table_shift;
+    int32_t* page_valid_len;
+    uint8_t* pages;
+    int64_t page_stride;
+    int32_t head_rows;        // 2 * num_kv_heads: K and V blocks of a page
+    int32_t row_bytes;
+    int32_t block_size;
+    int32_t pcp, interleave, max_local_blocks, num_pages;
+    int64_t num_tokens;
+    int32_t scan;             // find each page's filled slots in the table (else clear whole pages)
+};
+// Slots that the first num_tokens positions fill of table entry `entry`.
+__device__ __forceinline__ int filled_slots(const FillArgs& a, int entry) {
+    const int rank = entry / a.max_local_blocks;
+    const int64_t below = paging::owned_below(a.num_tokens, rank, a.pcp, a.interleave);
+    const int64_t n = below - (int64_t)(entry - rank * a.max_local_blocks) * a.block_size;
+    return (int)(n < 0 ? 0 : n > a.block_size ? a.block_size : n);
+}
+
+// Everything of a fresh pool that filling positions [0, num_tokens) does not
+// write: page blockIdx.x's slots past the ones its table entries fill (every
+// slot of a page that no entry names), by gridDim.y workgroups a page; and the
+// valid lengths of the entries, in closed form.  Must precede the write.  Every
+// workgroup looks through the whole table for its page: few thousand entries
+// from L2, against a pool cleared and written twice (the full 64-rank history:
+// 3 us here, 19 us to clear its 134 MB first); beyond kMaxScan (page, entry)
+// pairs the host asks for whole pages (scan 0).
+constexpr int64_t kMaxScan = 1ll << 24;
+__global__ void __launch_bounds__(kThreads) fill_rest_kernel(FillArgs a) {
+    __shared__ int most[kThreads / 64];
+    const int page = blockIdx.x, entries = a.pcp * a.max_local_blocks;
+    const int64_t part = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, parts = (int64_t)gridDim.x * gridDim.y;
+    for (int64_t e = part * kThreads + threadIdx.x; e < entries; e += parts * kThreads) {
+        const int pg = table_page(a.block_table, (int)e, a.table_shift);
+        a.page_valid_len[e] = (unsigned)pg < (unsigned)a.num_pages ? filled_slots(a, (int)e) : 0;
+    }
+    int n = 0;
+    for (int e = threadIdx.x; a.scan && e < entries; e += kThreads)
+        if (table_page(a.block_table, e, a.table_shift) == page) n = max(n, filled_slots(a, e));
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) n = max(n, __shfl_xor(n, off));
+    if ((threadIdx.x & 63) == 0) most[threadIdx.x >> 6] = n;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) n = max(n, most[w]);
+    // 16-byte chunks past slot n of each of the page's K and V blocks
+    const int per_block = (a.block_size - n) * (a.row_bytes / 16);
+    if (per_block == 0) return;
+    uint8_t* const base = a.pages + (int64_t)page * a.page_stride;
+    const int64_t block_bytes = (int64_t)a.block_size * a.row_bytes, skip = (int64_t)n * a.row_bytes;
+    const int64_t total = (int64_t)a.head_rows * per_block;
+    for (int64_t i = (int64_t)blockIdx.y * kThreads + threadIdx.x; i < total; i += (int64_t)gridDim.y * kThreads) {
+        const int b = (int)(i / per_block);
+        *(v4i*)(base + b * block_bytes + skip + (i - (int64_t)b * per_block) * 16) = v4i{0, 0, 0, 0};
+    }
+}
+
 // max |x| over n bf16 values into *out (as the bits of a non-negative float,
 // ordered like unsigned integers); *out is cleared first by init_kernel.
-__global__ void absmax_init_kernel(uint32_t* out) { *out = 0u; }
+__global__ void absmax_init_kernel(uint32_t* out) { out[threadIdx.x] = 0u; }
 
 // |x| of the two bf16 values of a dword, as their 15-bit magnitude patterns.
 // Non-negative IEEE values order like their bit patterns, and every NaN
@@ -206,8 +281,13 @@ __device__ __forceinline__ uint32_t abs_bits_max(uint32_t m, uint32_t word) {
 
 // Workgroup b reduces the contiguous span [b * span, (b + 1) * span) with
 // four 16-byte loads in flight per thread, then one atomic per workgroup.
-__global__ void __launch_bounds__(kThreads) absmax_kernel(const uint16_t* x, int64_t n, int64_t span,
-                                                          uint32_t* out) {
+// Grid y: x, or x and then `second` (of n values too, into out[1]).
+__global__ void __launch_bounds__(kThreads) absmax_kernel(const uint16_t* x, const uint16_t* second, int64_t n,
+                                                          int64_t span, uint32_t* out) {
+    if (blockIdx.y) {
+        x = second;
+        ++out;
+    }
     constexpr int kVec = 8, kUnroll = 4, kStep = kThreads * kVec;
     __shared__ uint32_t partial[kThreads / 64];
     const int64_t begin = (int64_t)blockIdx.x * span;

@@ -453,6 +453,129 @@ inline int32_t history_one_pass(const pcpa_params* p, const void* q, const void*
     return history_launch(p, 1, q, kv_pages, block_table, page_valid_len, out, lse, nullptr, 0, stream, &lease);
 }
 
+// max |x| (and |y|, of n values too, into amax[1]) of bf16 values.
+inline int32_t absmax(const void* x, const void* y, int64_t n, float* amax, hipStream_t stream) {
+    if (!x || !amax) return PCPA_ERR_NULL_POINTER;
+    if (n < 0) return PCPA_ERR_BAD_SHAPE;
+    if ((((uintptr_t)x | (uintptr_t)y) & 15u) || ((uintptr_t)amax & 3u)) return PCPA_ERR_MISALIGNED;
+    hipLaunchKernelGGL(cache::absmax_init_kernel, dim3(1), dim3(y ? 2 : 1), 0, stream, (uint32_t*)amax);
+    if (hipGetLastError() != hipSuccess) return PCPA_ERR_LAUNCH;
+    if (n == 0) return PCPA_OK;
+    // spans of whole 8-element groups (the span start stays 16-byte aligned),
+    // at least 32 KB each, at most 256 workgroups (one per CU: a 134 MB
+    // tensor then reads at 5.8 TB/s, against 3.7 TB/s with 2048 workgroups)
+    constexpr int64_t kMinSpan = 16384;
+    int64_t span = (n + 255) / 256;
+    span = span < kMinSpan ? kMinSpan : (span + 7) / 8 * 8;
+    const unsigned blocks = (unsigned)((n + span - 1) / span);
+    hipLaunchKernelGGL(cache::absmax_kernel, dim3(blocks, y ? 2 : 1), dim3(cache::kThreads), 0, stream,
+                       (const uint16_t*)x, (const uint16_t*)y, n, span, (uint32_t*)amax);
+    return hipGetLastError() == hipSuccess ? PCPA_OK : PCPA_ERR_LAUNCH;
+}
+
+// pcpa_kv_cache_write, or (fill) pcpa_kv_cache_fill: from position 0 into a
+// pool whose other slots are cleared, the lengths set rather than raised and
+// the e4m3 scales optionally taken from `amax`.
+inline int32_t cache_write(const pcpa_params* p, int32_t interleave, int64_t first_pos, int32_t num_tokens,
+                           const void* k, const void* v, const void* block_table, void* kv_pages,
+                           int32_t* page_valid_len, bool fill, const float* amax, void* stream) {
+    const int32_t st = pcpa_check_params(p);
+    if (st != PCPA_OK) return st;
+    if (!k || !v || !block_table || !kv_pages) return PCPA_ERR_NULL_POINTER;
+    if (interleave <= 0 || first_pos < 0 || num_tokens < 0) return PCPA_ERR_BAD_SHAPE;
+    if (((uintptr_t)k | (uintptr_t)v | (uintptr_t)kv_pages) & 15u) return PCPA_ERR_MISALIGNED;
+    if (((uintptr_t)block_table | (uintptr_t)page_valid_len) & 3u) return PCPA_ERR_MISALIGNED;
+    if ((p->flags & PCPA_FLAG_TABLE_INT64) && ((uintptr_t)block_table & 7u)) return PCPA_ERR_MISALIGNED;
+    if (num_tokens == 0 && !fill) return PCPA_OK;
+    // Every position must have a cache block: local index < max_local_blocks *
+    // block_size.  The local index grows with the position for each owner
+    // rank, so the largest one is among the last pcp_size * interleave
+    // positions of the range.
+    const int64_t capacity = (int64_t)p->max_local_blocks * p->block_size;  // per rank
+    const int64_t last = first_pos + num_tokens - 1;
+    const int64_t round_len = (int64_t)p->pcp_size * interleave;
+    for (int64_t pos = last; pos >= first_pos && pos > last - round_len; --pos) {
+        const int64_t chunk = pos / interleave;
+        if ((chunk / p->pcp_size) * interleave + pos % interleave >= capacity) return PCPA_ERR_BAD_SHAPE;
+    }
+    const int64_t chunks = (int64_t)p->num_kv_heads * num_tokens * (p->head_dim / 8);
+    if (last >= INT32_MAX || chunks > INT32_MAX || (int64_t)p->pcp_size * capacity > INT32_MAX)
+        return PCPA_ERR_TOO_LARGE;
+
+    const bool fp8 = p->kv_dtype == PCPA_DTYPE_FP8_E4M3FN;
+    const int64_t es = fp8 ? 1 : 2;
+    cache::WriteArgs a;
+    a.k = (const uint8_t*)k;
+    a.v = (const uint8_t*)v;
+    a.block_table = (const int32_t*)block_table;
+    a.table_shift = (p->flags & PCPA_FLAG_TABLE_INT64) ? 1 : 0;
+    a.page_valid_len = fill ? nullptr : page_valid_len;
+    a.pages = (uint8_t*)kv_pages;
+    a.amax = fp8 ? amax : nullptr;
+    a.head_stride = (int64_t)p->block_size * p->head_dim * es;
+    a.v_offset = (int64_t)p->num_kv_heads * a.head_stride;
+    a.page_stride = 2 * a.v_offset;
+    a.chunks_per_row = cache::make_fastdiv((uint32_t)(p->head_dim / 8));
+    a.interleave = cache::make_fastdiv((uint32_t)interleave);
+    a.pcp = cache::make_fastdiv((uint32_t)p->pcp_size);
+    a.block = cache::make_fastdiv((uint32_t)p->block_size);
+    auto log2_of = [](uint32_t x) -> int { return (x & (x - 1)) ? -1 : __builtin_ctz(x); };
+    const int l_cpr = log2_of((uint32_t)(p->head_dim / 8)), l_il = log2_of((uint32_t)interleave);
+    const int l_pcp = log2_of((uint32_t)p->pcp_size), l_blk = log2_of((uint32_t)p->block_size);
+    const bool pow2 = l_cpr >= 0 && l_il >= 0 && l_pcp >= 0 && l_blk >= 0;
+    a.log2_cpr = pow2 ? l_cpr : 0;
+    a.log2_il = pow2 ? l_il : 0;
+    a.log2_pcp = pow2 ? l_pcp : 0;
+    a.log2_block = pow2 ? l_blk : 0;
+    a.num_tokens = (uint32_t)num_tokens;
+    a.first_pos = (uint32_t)first_pos;
+    const int64_t next_chunk = (int64_t)(p->pcp_size - 1) * interleave + 1;
+    a.next_chunk = (uint32_t)(next_chunk < (1ll << 31) ? next_chunk : (1ll << 31));
+    a.max_local_blocks = p->max_local_blocks;
+    a.num_pages = p->num_pages;
+    a.head_dim = p->head_dim;
+    a.k_scale = p->k_scale;
+    a.v_scale = p->v_scale;
+    a.k_rcp = 1.f / p->k_scale;
+    a.v_rcp = 1.f / p->v_scale;
+    a.fast_div = cache::div_rn_covers(p->k_scale) && cache::div_rn_covers(p->v_scale) ? 1 : 0;
+    const uint32_t row_chunks = (uint32_t)num_tokens * (uint32_t)(p->head_dim / 8);
+    const dim3 grid((row_chunks + cache::kThreads - 1) / cache::kThreads, p->num_kv_heads);
+    const dim3 block(cache::kThreads);
+    const hipStream_t hs = (hipStream_t)stream;
+    if (fill) {
+        cache::FillArgs f;
+        f.block_table = a.block_table;
+        f.table_shift = a.table_shift;
+        f.page_valid_len = page_valid_len;
+        f.pages = a.pages;
+        f.page_stride = a.page_stride;
+        f.head_rows = 2 * p->num_kv_heads;
+        f.row_bytes = (int32_t)(p->head_dim * es);
+        f.block_size = p->block_size;
+        f.pcp = p->pcp_size;
+        f.interleave = interleave;
+        f.max_local_blocks = p->max_local_blocks;
+        f.num_pages = p->num_pages;
+        f.num_tokens = num_tokens;
+        f.scan = (int64_t)p->num_pages * p->pcp_size * p->max_local_blocks <= cache::kMaxScan;
+        // workgroups for the whole GPU even over few pages
+        const unsigned per_page = p->num_pages >= 1024 ? 1 : (1024 + p->num_pages - 1) / p->num_pages;
+        hipLaunchKernelGGL(cache::fill_rest_kernel, dim3(p->num_pages, per_page), dim3(cache::kThreads), 0, hs, f);
+        if (hipGetLastError() != hipSuccess) return PCPA_ERR_LAUNCH;
+        if (num_tokens == 0) return PCPA_OK;
+    }
+    if (fp8 && pow2)
+        hipLaunchKernelGGL((cache::kv_write_kernel<true, true>), grid, block, 0, hs, a, row_chunks);
+    else if (fp8)
+        hipLaunchKernelGGL((cache::kv_write_kernel<true, false>), grid, block, 0, hs, a, row_chunks);
+    else if (pow2)
+        hipLaunchKernelGGL((cache::kv_write_kernel<false, true>), grid, block, 0, hs, a, row_chunks);
+    else
+        hipLaunchKernelGGL((cache::kv_write_kernel<false, false>), grid, block, 0, hs, a, row_chunks);
+    return hipGetLastError() == hipSuccess ? PCPA_OK : PCPA_ERR_LAUNCH;
+}
+
 }  // namespace pcpa
 
 extern "C" {
@@ -592,101 +715,28 @@ int32_t pcpa_current_attention(const pcpa_params* p, int32_t interleave, const v
 }
 
 int32_t pcpa_absmax_bf16(const void* x, int64_t n, float* amax, void* stream) {
-    if (!x || !amax) return PCPA_ERR_NULL_POINTER;
-    if (n < 0) return PCPA_ERR_BAD_SHAPE;
-    if (((uintptr_t)x & 15u) || ((uintptr_t)amax & 3u)) return PCPA_ERR_MISALIGNED;
-    hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(pcpa::cache::absmax_init_kernel, dim3(1), dim3(1), 0, st, (uint32_t*)amax);
-    if (hipGetLastError() != hipSuccess) return PCPA_ERR_LAUNCH;
-    if (n == 0) return PCPA_OK;
-    // spans of whole 8-element groups (the span start stays 16-byte aligned),
-    // at least 32 KB each, at most 256 workgroups (one per CU: a 134 MB
-    // tensor then reads at 5.8 TB/s, against 3.7 TB/s with 2048 workgroups)
-    constexpr int64_t kMinSpan = 16384;
-    int64_t span = (n + 255) / 256;
-    span = span < kMinSpan ? kMinSpan : (span + 7) / 8 * 8;
-    const unsigned blocks = (unsigned)((n + span - 1) / span);
-    hipLaunchKernelGGL(pcpa::cache::absmax_kernel, dim3(blocks), dim3(pcpa::cache::kThreads), 0, st,
-                       (const uint16_t*)x, n, span, (uint32_t*)amax);
-    return hipGetLastError() == hipSuccess ? PCPA_OK : PCPA_ERR_LAUNCH;
+    return pcpa::absmax(x, nullptr, n, amax, (hipStream_t)stream);
+}
+
+int32_t pcpa_absmax_pair_bf16(const void* x, const void* y, int64_t n, float* amax, void* stream) {
+    if (!y) return PCPA_ERR_NULL_POINTER;
+    return pcpa::absmax(x, y, n, amax, (hipStream_t)stream);
 }
 
 int32_t pcpa_kv_cache_write(const pcpa_params* p, int32_t interleave, int64_t first_pos, int32_t num_tokens,
                             const void* k, const void* v, const void* block_table, void* kv_pages,
                             int32_t* page_valid_len, void* stream) {
-    const int32_t st = pcpa_check_params(p);
-    if (st != PCPA_OK) return st;
-    if (!k || !v || !block_table || !kv_pages) return PCPA_ERR_NULL_POINTER;
-    if (interleave <= 0 || first_pos < 0 || num_tokens < 0) return PCPA_ERR_BAD_SHAPE;
-    if (((uintptr_t)k | (uintptr_t)v | (uintptr_t)kv_pages) & 15u) return PCPA_ERR_MISALIGNED;
-    if (((uintptr_t)block_table | (uintptr_t)page_valid_len) & 3u) return PCPA_ERR_MISALIGNED;
-    if ((p->flags & PCPA_FLAG_TABLE_INT64) && ((uintptr_t)block_table & 7u)) return PCPA_ERR_MISALIGNED;
-    if (num_tokens == 0) return PCPA_OK;
-    // Every position must have a cache block: local index < max_local_blocks *
-    // block_size.  The local index grows with the position for each owner
-    // rank, so the largest one is among the last pcp_size * interleave
-    // positions of the range.
-    const int64_t capacity = (int64_t)p->max_local_blocks * p->block_size;  // per rank
-    const int64_t last = first_pos + num_tokens - 1;
-    const int64_t round_len = (int64_t)p->pcp_size * interleave;
-    for (int64_t pos = last; pos >= first_pos && pos > last - round_len; --pos) {
-        const int64_t chunk = pos / interleave;
-        if ((chunk / p->pcp_size) * interleave + pos % interleave >= capacity) return PCPA_ERR_BAD_SHAPE;
-    }
-    const int64_t chunks = (int64_t)p->num_kv_heads * num_tokens * (p->head_dim / 8);
-    if (last >= INT32_MAX || chunks > INT32_MAX || (int64_t)p->pcp_size * capacity > INT32_MAX)
-        return PCPA_ERR_TOO_LARGE;
+    return pcpa::cache_write(p, interleave, first_pos, num_tokens, k, v, block_table, kv_pages, page_valid_len, false,
+                             nullptr, stream);
+}
 
-    const bool fp8 = p->kv_dtype == PCPA_DTYPE_FP8_E4M3FN;
-    const int64_t es = fp8 ? 1 : 2;
-    pcpa::cache::WriteArgs a;
-    a.k = (const uint8_t*)k;
-    a.v = (const uint8_t*)v;
-    a.block_table = (const int32_t*)block_table;
-    a.table_shift = (p->flags & PCPA_FLAG_TABLE_INT64) ? 1 : 0;
-    a.page_valid_len = page_valid_len;
-    a.pages = (uint8_t*)kv_pages;
-    a.head_stride = (int64_t)p->block_size * p->head_dim * es;
-    a.v_offset = (int64_t)p->num_kv_heads * a.head_stride;
-    a.page_stride = 2 * a.v_offset;
-    a.chunks_per_row = pcpa::cache::make_fastdiv((uint32_t)(p->head_dim / 8));
-    a.interleave = pcpa::cache::make_fastdiv((uint32_t)interleave);
-    a.pcp = pcpa::cache::make_fastdiv((uint32_t)p->pcp_size);
-    a.block = pcpa::cache::make_fastdiv((uint32_t)p->block_size);
-    auto log2_of = [](uint32_t x) -> int { return (x & (x - 1)) ? -1 : __builtin_ctz(x); };
-    const int l_cpr = log2_of((uint32_t)(p->head_dim / 8)), l_il = log2_of((uint32_t)interleave);
-    const int l_pcp = log2_of((uint32_t)p->pcp_size), l_blk = log2_of((uint32_t)p->block_size);
-    const bool pow2 = l_cpr >= 0 && l_il >= 0 && l_pcp >= 0 && l_blk >= 0;
-    a.log2_cpr = pow2 ? l_cpr : 0;
-    a.log2_il = pow2 ? l_il : 0;
-    a.log2_pcp = pow2 ? l_pcp : 0;
-    a.log2_block = pow2 ? l_blk : 0;
-    a.num_tokens = (uint32_t)num_tokens;
-    a.first_pos = (uint32_t)first_pos;
-    const int64_t next_chunk = (int64_t)(p->pcp_size - 1) * interleave + 1;
-    a.next_chunk = (uint32_t)(next_chunk < (1ll << 31) ? next_chunk : (1ll << 31));
-    a.max_local_blocks = p->max_local_blocks;
-    a.num_pages = p->num_pages;
-    a.head_dim = p->head_dim;
-    a.k_scale = p->k_scale;
-    a.v_scale = p->v_scale;
-    a.k_rcp = 1.f / p->k_scale;
-    a.v_rcp = 1.f / p->v_scale;
-    auto div_ok = [](float d) { return d >= 0x1p-80f && d <= 0x1p126f; };
-    a.fast_div = div_ok(p->k_scale) && div_ok(p->v_scale) ? 1 : 0;
-    const uint32_t row_chunks = (uint32_t)num_tokens * (uint32_t)(p->head_dim / 8);
-    const dim3 grid((row_chunks + pcpa::cache::kThreads - 1) / pcpa::cache::kThreads, p->num_kv_heads);
-    const dim3 block(pcpa::cache::kThreads);
-    const hipStream_t hs = (hipStream_t)stream;
-    if (fp8 && pow2)
-        hipLaunchKernelGGL((pcpa::cache::kv_write_kernel<true, true>), grid, block, 0, hs, a, row_chunks);
-    else if (fp8)
-        hipLaunchKernelGGL((pcpa::cache::kv_write_kernel<true, false>), grid, block, 0, hs, a, row_chunks);
-    else if (pow2)
-        hipLaunchKernelGGL((pcpa::cache::kv_write_kernel<false, true>), grid, block, 0, hs, a, row_chunks);
-    else
-        hipLaunchKernelGGL((pcpa::cache::kv_write_kernel<false, false>), grid, block, 0, hs, a, row_chunks);
-    return hipGetLastError() == hipSuccess ? PCPA_OK : PCPA_ERR_LAUNCH;
+int32_t pcpa_kv_cache_fill(const pcpa_params* p, int32_t interleave, int32_t num_tokens, const void* k, const void* v,
+                           const float* amax, const void* block_table, void* kv_pages, int32_t* page_valid_len,
+                           void* stream) {
+    if (!page_valid_len) return PCPA_ERR_NULL_POINTER;
+    if ((uintptr_t)amax & 3u) return PCPA_ERR_MISALIGNED;
+    return pcpa::cache_write(p, interleave, 0, num_tokens, k, v, block_table, kv_pages, page_valid_len, true, amax,
+                             stream);
 }
 
 int32_t pcpa_block_mask_valid_len(const void* mask, int32_t pcp_size, int32_t max_local_blocks, int32_t block_size,

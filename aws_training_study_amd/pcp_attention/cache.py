@@ -21,14 +21,20 @@ from .inputs import per_tensor_scale
 from .kernel import _KV_DTYPE_CODES, _torch_kv_dtype
 
 
+def _check_absmax(x) -> None:
+    import torch
+
+    if not x.is_cuda or x.dtype != torch.bfloat16 or not x.is_contiguous():
+        raise ValueError("absmax expects a contiguous bfloat16 GPU tensor")
+
+
 def absmax(x):
     """max |x| of a contiguous BF16 GPU tensor, as a 0-d float32 GPU tensor (HIP reduction)."""
     import torch
 
     from .. import _native
 
-    if not x.is_cuda or x.dtype != torch.bfloat16 or not x.is_contiguous():
-        raise ValueError("absmax expects a contiguous bfloat16 GPU tensor")
+    _check_absmax(x)
     lib = _native.load_library()
     out = torch.empty((), dtype=torch.float32, device=x.device)
     with torch.cuda.device(x.device):
@@ -81,6 +87,33 @@ class KVCacheWriter:
         )
         self._fast = None  # the native call, made by the first one
 
+    def _check_tokens(self, k, v) -> None:
+        import torch
+
+        cfg = self.config
+        shape = (cfg.num_kv_heads, k.shape[1] if k.ndim == 3 else -1, cfg.head_dim)
+        for name, t in (("k", k), ("v", v)):
+            if (t.ndim != 3 or tuple(t.shape) != shape or t.dtype != torch.bfloat16 or not t.is_contiguous()
+                    or not t.is_cuda):
+                raise ValueError(f"{name} must be a contiguous bfloat16 GPU tensor {shape}, got "
+                                 f"{t.dtype} {tuple(t.shape)}")
+        if v.device != k.device:
+            raise ValueError(f"v is on {v.device}, k on {k.device}: all tensors must share one GPU")
+        if k.shape[1] >= 2**31:
+            raise ValueError("num_tokens must be below 2^31 and first_pos non-negative")
+
+    def _check_tables(self, block_table, page_valid_len) -> None:
+        import torch
+
+        table_shape = (self.config.pcp_size, self.config.max_local_blocks)
+        for name, t, dtypes in (("block_table", block_table, (torch.int32, torch.int64)),
+                                ("page_valid_len", page_valid_len, (torch.int32,))):
+            if t is None:
+                continue
+            if tuple(t.shape) != table_shape or t.dtype not in dtypes or not t.is_contiguous() or not t.is_cuda:
+                raise ValueError(f"{name} must be a contiguous {' or '.join(str(d) for d in dtypes)} GPU tensor "
+                                 f"{table_shape}")
+
     def __call__(self, k, v, kv_pages, block_table, *, first_pos: int = 0, k_scale: float = 1.0,
                  v_scale: float = 1.0, page_valid_len: Optional[object] = None) -> None:
         if self._fast is None:
@@ -94,23 +127,11 @@ class KVCacheWriter:
         import torch
 
         cfg = self.config
-        shape = (cfg.num_kv_heads, k.shape[1] if k.ndim == 3 else -1, cfg.head_dim)
-        for name, t in (("k", k), ("v", v)):
-            if (t.ndim != 3 or tuple(t.shape) != shape or t.dtype != torch.bfloat16 or not t.is_contiguous()
-                    or not t.is_cuda):
-                raise ValueError(f"{name} must be a contiguous bfloat16 GPU tensor {shape}, got "
-                                 f"{t.dtype} {tuple(t.shape)}")
+        self._check_tokens(k, v)
         if (kv_pages.ndim != 2 or kv_pages.shape[1] != cfg.page_elements
                 or kv_pages.dtype != _torch_kv_dtype(cfg.kv_dtype) or not kv_pages.is_contiguous()):
             raise ValueError(f"kv_pages must be a contiguous {cfg.kv_dtype} [num_pages, {cfg.page_elements}] pool")
-        table_shape = (cfg.pcp_size, cfg.max_local_blocks)
-        for name, t, dtypes in (("block_table", block_table, (torch.int32, torch.int64)),
-                                ("page_valid_len", page_valid_len, (torch.int32,))):
-            if t is None:
-                continue
-            if tuple(t.shape) != table_shape or t.dtype not in dtypes or not t.is_contiguous() or not t.is_cuda:
-                raise ValueError(f"{name} must be a contiguous {' or '.join(str(d) for d in dtypes)} GPU tensor "
-                                 f"{table_shape}")
+        self._check_tables(block_table, page_valid_len)
         for name, t in (("v", v), ("kv_pages", kv_pages), ("block_table", block_table),
                         ("page_valid_len", page_valid_len)):
             if t is not None and t.device != k.device:
@@ -142,15 +163,41 @@ def build_page_pool(config: PCPAttentionConfig, k, v, block_table, *, kv_scale: 
     cfg = replace(config, backend="hip").validate()
     if kv_scale not in ("per_tensor", "none"):
         raise ValueError(f"kv_scale must be 'per_tensor' or 'none', got {kv_scale!r}")
-    k_scale = v_scale = 1.0
-    if cfg.kv_dtype == "fp8_e4m3fn" and kv_scale == "per_tensor":
-        # both reductions queued, then one synchronisation for the two scales
-        amax_k, amax_v = torch.stack([absmax(k), absmax(v)]).tolist()
-        k_scale, v_scale = per_tensor_scale(amax_k), per_tensor_scale(amax_v)
-    pool = torch.zeros((cfg.num_pages, cfg.page_elements), dtype=_torch_kv_dtype(cfg.kv_dtype), device=k.device)
-    valid = torch.zeros((cfg.pcp_size, cfg.max_local_blocks), dtype=torch.int32, device=k.device)
+    per_tensor = cfg.kv_dtype == "fp8_e4m3fn" and kv_scale == "per_tensor"
+    for x in (k, v) if per_tensor else ():
+        _check_absmax(x)
+    writer = KVCacheWriter(cfg)
     table = block_table.to(device=k.device, dtype=torch.int32).contiguous()
-    KVCacheWriter(cfg)(k, v, pool, table, k_scale=k_scale, v_scale=v_scale, page_valid_len=valid)
+    writer._check_tokens(k, v)
+    writer._check_tables(table, None)
+    pool = torch.empty((cfg.num_pages, cfg.page_elements), dtype=_torch_kv_dtype(cfg.kv_dtype), device=k.device)
+    valid = torch.empty((cfg.pcp_size, cfg.max_local_blocks), dtype=torch.int32, device=k.device)
+    params = writer._native.PcpaParams(num_pages=cfg.num_pages, k_scale=1.0, v_scale=1.0, **writer._static)
+    lib = writer._lib
+    with torch.cuda.device(k.device):
+        stream = torch.cuda.current_stream(k.device)
+        amax = None
+        if per_tensor:
+            # the kernels take the scales from the GPU; the host's copy leaves
+            # the stream ahead of the fill, which then runs while it returns
+            amax = torch.empty(2, dtype=torch.float32, device=k.device)
+            writer._native.check(lib.pcpa_absmax_pair_bf16(k.data_ptr(), v.data_ptr(), k.numel(), amax.data_ptr(),
+                                                           stream.cuda_stream))
+            host = torch.empty(2, dtype=torch.float32, pin_memory=True)
+            host.copy_(amax, non_blocking=True)
+            copied = torch.cuda.Event()
+            copied.record(stream)
+        writer._native.check(lib.pcpa_kv_cache_fill(
+            ctypes.byref(params), cfg.interleave_size, k.shape[1], k.data_ptr(), v.data_ptr(),
+            None if amax is None else amax.data_ptr(), table.data_ptr(), pool.data_ptr(), valid.data_ptr(),
+            stream.cuda_stream))
+    if not per_tensor:
+        return pool, 1.0, 1.0, valid
+    copied.synchronize()
+    k_scale, v_scale = (per_tensor_scale(x) for x in host.tolist())
+    # the launch checks of a write with these scales (an infinity in K or V)
+    params.k_scale, params.v_scale = k_scale, v_scale
+    writer._native.check(lib.pcpa_check_params(ctypes.byref(params)))
     return pool, k_scale, v_scale, valid
 
 

@@ -297,6 +297,24 @@ int32_t pcpa_kv_cache_write(const pcpa_params* params, int32_t interleave, int64
                             void* stream);
 
 /*
+ * Fill a fresh pool: pcpa_kv_cache_write of positions [0, num_tokens), and the
+ * rest of the pool cleared - every slot that no written token takes, in pages
+ * that the table names and in pages that it does not - so that kv_pages needs
+ * no initialisation.
+ *   page_valid_len  int32 [pcp_size, max_local_blocks], set (not raised): the
+ *                   tokens written to each entry's block, 0 for an entry
+ *                   outside [0, num_pages)
+ *   amax            optional device float[2], the largest |K| and |V| (what
+ *                   pcpa_absmax_pair_bf16 writes): an e4m3 pool then stores
+ *                   x / (amax / 448) (x itself where amax is 0 or NaN) instead
+ *                   of using params' scales, without a host round trip.
+ * num_tokens may be 0 (the pool is cleared).
+ */
+int32_t pcpa_kv_cache_fill(const pcpa_params* params, int32_t interleave, int32_t num_tokens,
+                           const void* k, const void* v, const float* amax, const void* block_table,
+                           void* kv_pages, int32_t* page_valid_len, void* stream);
+
+/*
  * max |x| over n bf16 values into *amax (device float): the amax of the
  * per-tensor e4m3 scale amax / 448 (the FP8 configurations' K/V
  * quantisation).  A NaN anywhere in x makes *amax NaN, as torch's
@@ -304,6 +322,8 @@ int32_t pcpa_kv_cache_write(const pcpa_params* params, int32_t interleave, int64
  * initialisation.
  */
 int32_t pcpa_absmax_bf16(const void* x, int64_t n, float* amax, void* stream);
+/* The same of two tensors of n values each, into amax[0] and amax[1]. */
+int32_t pcpa_absmax_pair_bf16(const void* x, const void* y, int64_t n, float* amax, void* stream);
 
 /*
  * The reference's runtime mask turned into per-page valid lengths on the GPU
