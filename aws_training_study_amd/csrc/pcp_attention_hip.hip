@@ -18,8 +18,9 @@
 //   * ovl::history_fwd_overlap<256, FAST, LSE, SPLIT> (overlap_kernel.hpp):
 //     the e4m3-MFMA path at head_dim 256, 8 waves x 32 rows, a two-stage
 //     in-wave pipeline with the two waves of a SIMD staggered by half a tile
-//     step; SPLIT walks one range of the table and writes a partial result
-//     for merge_splits_kernel.
+//     step (history_fwd_overlap_waves: 4 waves, for launches of few rows);
+//     SPLIT walks one range of the table and writes a partial result for
+//     merge_splits_kernel.
 // cache_kernels.hpp holds the KV-cache producer.
 //
 // Work decomposition

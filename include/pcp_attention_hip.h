@@ -59,7 +59,7 @@ extern "C" {
 
 /* params.flags bits. */
 /* Run both GEMMs as BF16 MFMAs even for an e4m3 cache: K/V are widened to
- * bf16 exactly while staged, Q and P stay bf16.  Half the MFMA rate, but no
+ * bf16 exactly as they are read from LDS, Q and P stay bf16.  Half the MFMA rate, but no
  * e4m3 rounding of Q and P.  Ignored for a bf16 cache. */
 #define PCPA_FLAG_BF16_MFMA 1u
 /* FP8 MFMA path at head_dim 256: compute the e4m3 probabilities with
