@@ -153,7 +153,7 @@ void* workspace_for(Call* c, void* stream, at::Tensor& hold) {
     return hold.data_ptr();
 }
 
-// (q, kv_pages, block_table, page_valid_len, k_scale, v_scale, out, return_lse)
+// (q, kv_pages, block_table, page_valid_len, k_scale, v_scale, out, return_lse) -> outputs or a status
 PyObject* history(Call* c, PyObject* const* a) {
     const at::Tensor *q = plain(a[0]), *kv = plain(a[1]), *table = plain(a[2]), *valid = plain(a[3]);
     const at::Tensor* given = a[6] == Py_None ? nullptr : plain(a[6]);
@@ -190,11 +190,11 @@ PyObject* history(Call* c, PyObject* const* a) {
     } else {
         status = launch([&] { return ((HistoryLse)c->fn)(&p, qp, kp, tp, vp, op, lse_ptr, stream); });
     }
-    if (status) GIVE_UP;
+    if (status) return PyLong_FromLong(status);
     return tensors(out, lse);
 }
 
-// (q, kv_current, hist_out, hist_lse, out, return_lse)
+// (q, kv_current, hist_out, hist_lse, out, return_lse) -> outputs or a status
 PyObject* current(Call* c, PyObject* const* a) {
     const at::Tensor *q = plain(a[0]), *kv = plain(a[1]);
     const at::Tensor* hist = a[2] == Py_None ? nullptr : plain(a[2]);
@@ -225,11 +225,11 @@ PyObject* current(Call* c, PyObject* const* a) {
     float* const lp = lse.defined() ? (float*)lse.data_ptr() : nullptr;
     const int32_t status =
         launch([&] { return ((Current)c->fn)(&p, c->interleave, qp, kp, hp, hl, op, lp, stream); });
-    if (status) GIVE_UP;
+    if (status) return PyLong_FromLong(status);
     return tensors(out, lse);
 }
 
-// (k, v, kv_pages, block_table, first_pos, k_scale, v_scale, page_valid_len) -> True
+// (k, v, kv_pages, block_table, first_pos, k_scale, v_scale, page_valid_len) -> status
 PyObject* write(Call* c, PyObject* const* a) {
     const at::Tensor *k = plain(a[0]), *v = plain(a[1]), *kv = plain(a[2]), *table = plain(a[3]);
     const at::Tensor* valid = a[7] == Py_None ? nullptr : plain(a[7]);
@@ -256,11 +256,10 @@ PyObject* write(Call* c, PyObject* const* a) {
     const int32_t status = launch([&] {
         return ((Write)c->fn)(&p, c->interleave, first, (int32_t)n, kp, vp, tp, pages, lens, stream);
     });
-    if (status) GIVE_UP;
-    Py_RETURN_TRUE;
+    return PyLong_FromLong(status);
 }
 
-// (first_pos, num_tokens, block_table, free_pages, free_count) -> True
+// (first_pos, num_tokens, block_table, free_pages, free_count) -> status
 PyObject* alloc(Call* c, PyObject* const* a) {
     const at::Tensor *table = plain(a[2]), *pages = plain(a[3]), *count = plain(a[4]);
     int64_t first, n;
@@ -278,8 +277,7 @@ PyObject* alloc(Call* c, PyObject* const* a) {
     int32_t* const cp = (int32_t*)count->data_ptr();
     const int32_t status =
         launch([&] { return ((Alloc)c->fn)(&p, c->interleave, first, (int32_t)n, tp, pp, cp, stream); });
-    if (status) GIVE_UP;
-    Py_RETURN_TRUE;
+    return PyLong_FromLong(status);
 }
 
 template <PyObject* (*F)(Call*, PyObject* const*), Py_ssize_t N>

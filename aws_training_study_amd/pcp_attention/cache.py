@@ -121,9 +121,11 @@ class KVCacheWriter:
             self._fast = self._native.fast_calls().make(
                 "write", bytes(params), self.config.kv_dtype == "fp8_e4m3fn", self.config.interleave_size,
                 self._native.function_address(self._lib.pcpa_kv_cache_write))
-        if self._fast(k, v, kv_pages, block_table, first_pos, k_scale, v_scale, page_valid_len):
+        status = self._fast(k, v, kv_pages, block_table, first_pos, k_scale, v_scale, page_valid_len)
+        if status is not None:
+            self._native.check(status)
             return
-        # not the common form, or an error
+        # not the common form
         import torch
 
         cfg = self.config
@@ -250,9 +252,11 @@ class PageAllocator:
             self._fast = self._native.fast_calls().make(
                 "alloc", bytes(self._params), False, self.config.interleave_size,
                 self._native.function_address(self._lib.pcpa_page_alloc))
-        if self._fast(first_pos, num_tokens, block_table, self.free_pages, self.free_count):
+        status = self._fast(first_pos, num_tokens, block_table, self.free_pages, self.free_count)
+        if status is not None:
+            self._native.check(status)
             return
-        # not the common form, or an error
+        # not the common form
         import torch
 
         cfg = self.config

@@ -90,9 +90,11 @@ class CurrentAttentionKernel:
                 "current", bytes(self._launch_params), False, self.config.interleave_size,
                 self._native.function_address(self._lib.pcpa_current_attention))
         result = self._fast(q, kv_current, hist_out, hist_lse, out, return_lse)
+        if type(result) is int:  # the status of a launch that failed
+            self._native.check(result)
         if result is not None:
             return result
-        # not the common form, or an error
+        # not the common form
         import torch
 
         cfg = self.config

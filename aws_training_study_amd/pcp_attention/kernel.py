@@ -218,14 +218,16 @@ class HistoryAttentionKernel:
         workspace=None,
     ):
         if page_valid_len is not None and block_valid_mask is None and workspace is None:
-            # the common form of the call, checked and launched natively;
-            # None: not that form (or an error), which the rest of this
-            # function sees to
+            # the common form of the call, checked and launched natively (an
+            # int: the status of a launch that failed); None: not that form,
+            # which the rest of this function sees to
             plan = self._plans.get((precision, exp2, splits))
             if plan is None:
                 plan = self._plan(precision, exp2, splits, page_valid_len)
             if plan is not None:
                 result = plan(q, kv_pages, block_table, page_valid_len, k_scale, v_scale, out, return_lse)
+                if type(result) is int:
+                    self._native.check(result)
                 if result is not None:
                     return result
         import torch

@@ -6,9 +6,12 @@ general path: same results, same conversions, same errors.
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
+from aws_training_study_amd import _native
 from aws_training_study_amd.pcp_attention import (
     KVCacheWriter,
     PageAllocator,
@@ -112,3 +115,39 @@ def test_current_and_cache_calls(cuda_device):
         writer(x, x, a[1], a[2], first_pos=400)
     with pytest.raises(RuntimeError, match="BAD_SHAPE"):
         a[0].allocate(400, 300, a[2])
+
+
+# Pointer-sized arguments of the C entries behind the native calls.
+C_ENTRY_ARGS = {"pcpa_history_attention_lse": 8, "pcpa_history_attention_split": 11, "pcpa_current_attention": 9,
+                "pcpa_kv_cache_write": 10, "pcpa_page_alloc": 8}
+
+
+@pytest.mark.parametrize("entry", sorted(C_ENTRY_ARGS))
+def test_a_failed_launch_is_raised_and_not_made_again(entry, cuda_device, monkeypatch):
+    """A status of the C entry is the call's error: kernels of it may be
+    queued, so that the general path must not make the call a second time."""
+    cfg, q, pool, table, valid, k_scale, v_scale = _case(cuda_device)
+    calls = []
+
+    def fail(*args):
+        calls.append(entry)
+        return next(code for code, name in _native.STATUS_NAMES.items() if name == "PCPA_ERR_LAUNCH")
+
+    c_fail = ctypes.CFUNCTYPE(ctypes.c_int32, *[ctypes.c_void_p] * C_ENTRY_ARGS[entry])(fail)
+    monkeypatch.setattr(_native, "function_address", lambda fn: ctypes.cast(c_fail, ctypes.c_void_p).value)
+    x = torch.randn((2, 300, 64), device=cuda_device, dtype=torch.bfloat16)
+    zeros = torch.zeros_like(table)
+    with pytest.raises(_native.PcpaError, match="LAUNCH"):
+        if entry.startswith("pcpa_history"):
+            splits = 1 if entry.endswith("lse") else 2
+            make_history_attention_kernel(cfg)(q, pool, table, page_valid_len=valid, k_scale=k_scale,
+                                               v_scale=v_scale, precision="fp8", splits=splits)
+        elif entry == "pcpa_current_attention":
+            CurrentAttentionKernel(cfg)(q, x[None, :, :128].expand(2, -1, -1, -1).contiguous())
+        elif entry == "pcpa_kv_cache_write":
+            KVCacheWriter(cfg)(x, x, pool, table, page_valid_len=zeros)
+        else:
+            PageAllocator(cfg, cuda_device).allocate(0, 300, zeros - 1)
+    assert calls == [entry]
+    torch.cuda.synchronize()
+    assert int(zeros.sum()) == 0
