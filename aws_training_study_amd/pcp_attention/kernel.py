@@ -522,7 +522,7 @@ class HistoryAttentionKernel:
                 self._split_ws.clear()
             ws = torch.empty(max(size, 16), dtype=torch.uint8, device=device)
             self._split_ws[key] = ws
-            for plan in self._plans.values():
+            for plan in list(self._plans.values()):  # (other threads may add plans meanwhile)
                 plan.forget()  # workspaces dropped here are dropped there too
         return ws
 
