@@ -221,9 +221,13 @@ class HistoryAttentionKernel:
             # the common form of the call, checked and launched natively (an
             # int: the status of a launch that failed); None: not that form,
             # which the rest of this function sees to
-            plan = self._plans.get((precision, exp2, splits))
-            if plan is None:
-                plan = self._plan(precision, exp2, splits, page_valid_len)
+            try:
+                plan = self._plans.get((precision, exp2, splits))
+            except TypeError:  # an option that cannot be looked up
+                plan = None
+            else:
+                if plan is None:
+                    plan = self._plan(precision, exp2, splits, page_valid_len)
             if plan is not None:
                 result = plan(q, kv_pages, block_table, page_valid_len, k_scale, v_scale, out, return_lse)
                 if type(result) is int:
@@ -340,11 +344,13 @@ class HistoryAttentionKernel:
 
     def _plan(self, precision, exp2, splits, page_valid_len):
         """The native call of this form on the lengths' GPU, kept; ``None`` for
-        lengths that are not on a GPU and for options the general path refuses."""
+        lengths that are not on a GPU and for options the general path converts
+        or refuses."""
         import weakref
 
-        if (precision not in PRECISIONS or exp2 not in EXP2_MODES or not (splits == "auto" or type(splits) is int)
-                or not getattr(page_valid_len, "is_cuda", False)):
+        counted = type(splits) is int and 1 <= splits <= self._native.MAX_SPLITS
+        if (not (counted or type(splits) is str and splits == "auto") or precision not in PRECISIONS
+                or exp2 not in EXP2_MODES or not getattr(page_valid_len, "is_cuda", False)):
             return None
         device = page_valid_len.device
         bf16_mfma, guard = self._modes[precision]

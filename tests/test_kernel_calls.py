@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -31,3 +32,25 @@ def test_workspaces_while_another_thread_makes_plans(kernel):
     kernel._plans["a"], kernel._plans["b"] = Plan("a"), Plan("b")
     assert kernel._workspace(64, torch.device("cpu"), 7).numel() == 64
     assert forgotten == ["a", "b"]
+
+
+@pytest.mark.parametrize("option,value,message", [
+    ("precision", ["auto"], "precision must be one of"),
+    ("exp2", {"fast": 1}, "exp2 must be one of"),
+    # accepted values that cannot be looked up or kept as they are: on to the next check
+    ("splits", np.array(2), "q must be a GPU tensor"),
+    ("splits", 2.0, "q must be a GPU tensor"),
+    ("splits", -2**40, "q must be a GPU tensor"),
+    ("splits", 99, "q must be a GPU tensor"),
+])
+def test_options_are_checked_by_the_general_path(kernel, option, value, message):
+    """Looking up the native call neither refuses an option nor raises ahead
+    of the general path's checks, whatever the option's type or range."""
+
+    class OnGpu:  # lengths that say they are on a GPU, so that a plan is made if the options allow one
+        is_cuda, device = True, torch.device("cuda", 0)
+
+    kernel.split_count = lambda *_: 1  # (asks the device)
+    q = torch.zeros((2, 4, 64, 64), dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match=message):
+        kernel(q, None, None, page_valid_len=OnGpu(), **{option: value})
