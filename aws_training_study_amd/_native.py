@@ -123,6 +123,13 @@ def load_library() -> ctypes.CDLL:
             "(or aws_training_study_amd.build_native.build())"
         )
     lib = ctypes.CDLL(os.fspath(path))
+    missing = [name for name in EXPORTED_SYMBOLS if not hasattr(lib, name)]
+    version = None if "pcpa_abi_version" in missing else lib.pcpa_abi_version()  # (no arguments, returns int32)
+    if version != ABI_VERSION:
+        raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}; rebuild it")
+    if missing:
+        # entries are added without a new version: it covers what a C caller's params mean
+        raise RuntimeError(f"{path} lacks {', '.join(missing)}; rebuild it")
     lib.pcpa_abi_version.restype = ctypes.c_int32
     lib.pcpa_abi_version.argtypes = []
     lib.pcpa_status_string.restype = ctypes.c_char_p
@@ -177,9 +184,6 @@ def load_library() -> ctypes.CDLL:
     lib.pcpa_page_alloc.restype = ctypes.c_int32
     lib.pcpa_page_alloc.argtypes = [ctypes.POINTER(PcpaParams), ctypes.c_int32, ctypes.c_int64, ctypes.c_int32,
                                     ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
-    version = lib.pcpa_abi_version()
-    if version != ABI_VERSION:
-        raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}; rebuild it")
     _lib = lib
     return lib
 
