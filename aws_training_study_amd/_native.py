@@ -16,6 +16,8 @@ LIB_DIR = Path(__file__).resolve().parent / "_lib"
 LIB_NAME = "libpcp_attention_hip.so"
 
 ABI_VERSION = 3
+# What the entry points expect of the extension's calls (csrc/fast_calls.cpp).
+FAST_CALLS_VERSION = 2
 
 PCPA_OK = 0
 STATUS_NAMES = {
@@ -197,15 +199,24 @@ def fast_calls():
     if _fast_calls is None:
         import importlib.util
 
-        import torch  # noqa: F401  (its libraries hold the extension's symbols)
+        import torch  # (its libraries hold the extension's symbols)
 
-        path = Path(__file__).resolve().parent / "_lib" / "_pcpa_fast_calls.so"
+        path = LIB_DIR / "_pcpa_fast_calls.so"
         if not path.exists():
             raise RuntimeError(f"extension {path} is missing; build it with "
                                "`python -c 'import __graft_entry__ as g; g.build()'`")
         spec = importlib.util.spec_from_file_location("_pcpa_fast_calls", path)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
+        try:
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+        except ImportError as error:  # e.g. symbols of another torch build
+            raise RuntimeError(f"extension {path} does not load ({error}); rebuild it") from error
+        version = getattr(module, "version", None)
+        if version != FAST_CALLS_VERSION:
+            raise RuntimeError(f"{path} has version {version}, expected {FAST_CALLS_VERSION}; rebuild it")
+        if module.torch_version != torch.__version__:
+            raise RuntimeError(f"{path} was built for torch {module.torch_version}, this is {torch.__version__}; "
+                               "rebuild it")
         _fast_calls = module
     return _fast_calls
 

@@ -104,6 +104,7 @@ def fast_calls_command(output: Path = FAST_CALLS) -> list[str]:
         "-shared",
         "-fPIC",
         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f'-DPCPA_TORCH_VERSION="{torch.__version__}"',
         f"-I{INCLUDE_DIR}",
         f"-I{sysconfig.get_paths()['include']}",
         *[f"-I{path}" for path in cpp_extension.include_paths()],

@@ -26,6 +26,10 @@
 
 namespace {
 
+// What the calls take and return, checked when the module is loaded (as is
+// PCPA_TORCH_VERSION, the torch that the build line names).
+constexpr int kVersion = 2;
+
 PyObject* g_raw_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
 PyObject* g_device = nullptr;      // torch._C._cuda_getDevice
 
@@ -411,5 +415,12 @@ PyMODINIT_FUNC PyInit__pcpa_fast_calls(void) {
     g_device = PyObject_GetAttrString(c, "_cuda_getDevice");
     Py_DECREF(c);
     if (!g_raw_stream || !g_device) return nullptr;
-    return PyModule_Create(&module);
+    PyObject* const m = PyModule_Create(&module);
+    if (!m) return nullptr;
+    if (PyModule_AddIntConstant(m, "version", kVersion) < 0 ||
+        PyModule_AddStringConstant(m, "torch_version", PCPA_TORCH_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }
