@@ -489,15 +489,18 @@ inline int32_t cache_write(const pcpa_params* p, int32_t interleave, int64_t fir
     if ((p->flags & PCPA_FLAG_TABLE_INT64) && ((uintptr_t)block_table & 7u)) return PCPA_ERR_MISALIGNED;
     if (num_tokens == 0 && !fill) return PCPA_OK;
     // Every position must have a cache block: local index < max_local_blocks *
-    // block_size.  The local index grows with the position for each owner
-    // rank, so the largest one is among the last pcp_size * interleave
-    // positions of the range.
+    // block_size.  The largest local index of the range is the last position's
+    // or, if the chunk before it is another rank's chunk of the same round and
+    // the range reaches back to it, that of the chunk's end.  (Looking at the
+    // last pcp_size * interleave positions one by one took 7 us of host time a
+    // call for 1000 tokens of 16 ranks x 64, and seconds for the widest stripes.)
     const int64_t capacity = (int64_t)p->max_local_blocks * p->block_size;  // per rank
     const int64_t last = first_pos + num_tokens - 1;
-    const int64_t round_len = (int64_t)p->pcp_size * interleave;
-    for (int64_t pos = last; pos >= first_pos && pos > last - round_len; --pos) {
-        const int64_t chunk = pos / interleave;
-        if ((chunk / p->pcp_size) * interleave + pos % interleave >= capacity) return PCPA_ERR_BAD_SHAPE;
+    if (num_tokens > 0) {
+        const int64_t chunk = last / interleave, round = chunk / p->pcp_size;
+        const bool earlier = chunk > round * p->pcp_size && chunk * interleave > first_pos;
+        const int64_t slot = earlier ? interleave - 1 : last - chunk * interleave;
+        if (round * interleave + slot >= capacity) return PCPA_ERR_BAD_SHAPE;
     }
     const int64_t chunks = (int64_t)p->num_kv_heads * num_tokens * (p->head_dim / 8);
     if (last >= INT32_MAX || chunks > INT32_MAX || (int64_t)p->pcp_size * capacity > INT32_MAX)

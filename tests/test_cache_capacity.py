@@ -1,0 +1,58 @@
+"""Which positions the cache producer accepts, decided on the host.
+
+The calls here have 2^26 KV heads of head_dim 256, so that one token already
+holds more chunks than the producer indexes: a range that fits the cache is
+refused as too large (and none of them launches anything), one that does not
+fit as a bad shape.
+"""
+
+from __future__ import annotations
+
+import ctypes
+import random
+import time
+
+import pytest
+
+from aws_training_study_amd import _native
+
+BAD_SHAPE, TOO_LARGE = -3, -8
+
+
+def _write(pcp, interleave, blocks, block_size, first, tokens):
+    p = _native.PcpaParams(abi_version=_native.ABI_VERSION, pcp_size=pcp, num_q_heads=1 << 26, num_kv_heads=1 << 26,
+                           head_dim=256, local_q_len=1, block_size=block_size, max_local_blocks=blocks, num_pages=1,
+                           q_dtype=1, kv_dtype=1, out_dtype=1, softmax_scale=1.0, k_scale=1.0, v_scale=1.0, flags=0)
+    return _native.load_library().pcpa_kv_cache_write(ctypes.byref(p), interleave, first, tokens, 16, 16, 16, 16,
+                                                      None, None)
+
+
+def _fits(pcp, interleave, capacity, first, tokens):
+    """Every position of the range has a local index below the rank's capacity."""
+    return all(pos // interleave // pcp * interleave + pos % interleave < capacity
+               for pos in range(first, first + tokens))
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_ranges_at_the_capacity(seed):
+    rng = random.Random(seed)
+    seen = {BAD_SHAPE: 0, TOO_LARGE: 0}
+    for _ in range(400):
+        pcp, interleave = rng.choice([1, 2, 3, 4, 5, 16]), rng.choice([1, 3, 16, 48, 64, 100, 1000])
+        blocks, block_size = rng.choice([1, 2, 3]), rng.choice([64, 128, 192])
+        capacity = blocks * block_size
+        end = max(1, pcp * capacity + rng.randint(-3 * interleave, 3 * interleave * pcp))
+        tokens = rng.randint(1, min(end, rng.choice([1, 2, interleave + 1, 2 * pcp * interleave, end])))
+        status = _write(pcp, interleave, blocks, block_size, end - tokens, tokens)
+        fits = _fits(pcp, interleave, capacity, end - tokens, tokens)
+        assert status == (TOO_LARGE if fits else BAD_SHAPE), (pcp, interleave, capacity, end - tokens, tokens)
+        seen[status] += 1
+    assert min(seen.values()) >= 50
+
+
+def test_wide_stripes_are_decided_at_once():
+    """The decision's time does not grow with the stripe (2^31 positions one by one took 9 s)."""
+    start = time.perf_counter()
+    assert _write(4, 1 << 30, 1 << 11, 1 << 20, 0, 2**31 - 1) == TOO_LARGE
+    assert _write(4, 1 << 30, 1 << 9, 1 << 20, 0, 2**31 - 1) == BAD_SHAPE
+    assert time.perf_counter() - start < 1.0
