@@ -483,7 +483,8 @@ inline int32_t cache_write(const pcpa_params* p, int32_t interleave, int64_t fir
     const int32_t st = pcpa_check_params(p);
     if (st != PCPA_OK) return st;
     if (!k || !v || !block_table || !kv_pages) return PCPA_ERR_NULL_POINTER;
-    if (interleave <= 0 || first_pos < 0 || num_tokens < 0) return PCPA_ERR_BAD_SHAPE;
+    if (interleave <= 0 || first_pos < 0 || num_tokens < 0 || first_pos > INT64_MAX - num_tokens)
+        return PCPA_ERR_BAD_SHAPE;
     if (((uintptr_t)k | (uintptr_t)v | (uintptr_t)kv_pages) & 15u) return PCPA_ERR_MISALIGNED;
     if (((uintptr_t)block_table | (uintptr_t)page_valid_len) & 3u) return PCPA_ERR_MISALIGNED;
     if ((p->flags & PCPA_FLAG_TABLE_INT64) && ((uintptr_t)block_table & 7u)) return PCPA_ERR_MISALIGNED;
@@ -760,7 +761,8 @@ int32_t pcpa_page_alloc(const pcpa_params* p, int32_t interleave, int64_t first_
     const int32_t st = pcpa_check_params(p);
     if (st != PCPA_OK) return st;
     if (!block_table || !free_pages || !free_count) return PCPA_ERR_NULL_POINTER;
-    if (interleave <= 0 || first_pos < 0 || num_tokens < 0) return PCPA_ERR_BAD_SHAPE;
+    if (interleave <= 0 || first_pos < 0 || num_tokens < 0 || first_pos > INT64_MAX - num_tokens)
+        return PCPA_ERR_BAD_SHAPE;
     if (((uintptr_t)block_table | (uintptr_t)free_pages | (uintptr_t)free_count) & 3u) return PCPA_ERR_MISALIGNED;
     if ((p->flags & PCPA_FLAG_TABLE_INT64) && ((uintptr_t)block_table & 7u)) return PCPA_ERR_MISALIGNED;
     if (num_tokens == 0) return PCPA_OK;

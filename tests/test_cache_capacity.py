@@ -56,3 +56,20 @@ def test_wide_stripes_are_decided_at_once():
     assert _write(4, 1 << 30, 1 << 11, 1 << 20, 0, 2**31 - 1) == TOO_LARGE
     assert _write(4, 1 << 30, 1 << 9, 1 << 20, 0, 2**31 - 1) == BAD_SHAPE
     assert time.perf_counter() - start < 1.0
+
+
+@pytest.mark.parametrize("first,tokens", [(2**63 - 1, 1), (2**63 - 1, 2), (2**63 - 2, 2), (2**63 - 300, 2**31 - 1)])
+@pytest.mark.parametrize("entry", ["write", "alloc"])
+def test_positions_beyond_64_bits(entry, first, tokens):
+    """A range whose end is not an int64 fits no cache (the end wrapped
+    round: the allocator took it for an empty range, the producer's checks
+    were left to what the compiler made of the overflow)."""
+    p = _native.PcpaParams(abi_version=_native.ABI_VERSION, pcp_size=4, num_q_heads=8, num_kv_heads=2, head_dim=64,
+                           local_q_len=64, block_size=128, max_local_blocks=4, num_pages=16, q_dtype=1, kv_dtype=1,
+                           out_dtype=1, softmax_scale=1.0, k_scale=1.0, v_scale=1.0, flags=0)
+    lib = _native.load_library()
+    if entry == "write":
+        status = lib.pcpa_kv_cache_write(ctypes.byref(p), 16, first, tokens, 16, 16, 16, 16, None, None)
+    else:
+        status = lib.pcpa_page_alloc(ctypes.byref(p), 16, first, tokens, 16, 16, 16, None)
+    assert status == BAD_SHAPE
