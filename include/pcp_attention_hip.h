@@ -308,7 +308,8 @@ int32_t pcpa_kv_cache_write(const pcpa_params* params, int32_t interleave, int64
  *                   pcpa_absmax_pair_bf16 writes): an e4m3 pool then stores
  *                   x / (amax / 448) (x itself where amax is 0 or NaN) instead
  *                   of using params' scales, without a host round trip.
- * num_tokens may be 0 (the pool is cleared).
+ * num_tokens may be 0 (the pool is cleared; k and v must be non-null all the
+ * same).
  */
 int32_t pcpa_kv_cache_fill(const pcpa_params* params, int32_t interleave, int32_t num_tokens,
                            const void* k, const void* v, const float* amax, const void* block_table,

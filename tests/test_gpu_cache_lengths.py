@@ -58,7 +58,7 @@ def test_valid_lengths_of_ragged_ranges(pcp, il, block, kv_dtype, cuda_device):
 @pytest.mark.parametrize("kv_dtype,kv_scale", [("fp8_e4m3fn", "per_tensor"), ("fp8_e4m3fn", "none"), ("bfloat16", "none")])
 def test_fresh_pool_equals_a_write_into_zeros(pcp, il, block, kv_dtype, kv_scale, cuda_device):
     """build_page_pool clears only what it does not write: slots past a ragged
-    length, pages that the table names twice, not at all or with a hole."""
+    length and the pages of a hole in the table."""
     bucket = pcp * il * max(1, 2 * block // il)
     cfg = PCPAttentionConfig(pcp_size=pcp, current_len=pcp * il, max_history_len=bucket, actual_history_len=bucket,
                              block_size=block, interleave_size=il, num_q_heads=2, num_kv_heads=2, head_dim=64,
@@ -74,7 +74,7 @@ def test_fresh_pool_equals_a_write_into_zeros(pcp, il, block, kv_dtype, kv_scale
             k[0, 5, 5] = float("nan")  # an amax of NaN: unit scale
         for table in (identity, holes.int(), identity.flip(1).cpu()):
             # freed memory that is not zero, for the pool to land in
-            torch.full((cfg.num_pages, cfg.page_elements), 255, dtype=torch.uint8, device=cuda_device)
+            torch.full((cfg.num_pages, cfg.page_elements * dtype.itemsize), 255, dtype=torch.uint8, device=cuda_device)
             pool, k_scale, v_scale, valid = build_page_pool(cfg, k, v, table, kv_scale=kv_scale)
             want = torch.zeros((cfg.num_pages, cfg.page_elements), dtype=dtype, device=cuda_device)
             lens = torch.zeros((pcp, cfg.max_local_blocks), dtype=torch.int32, device=cuda_device)
