@@ -137,6 +137,14 @@ PyObject* tensors(const at::Tensor& out, const at::Tensor& lse) {
     return t;
 }
 
+// Forget the remembered workspaces.  Freeing a tensor can release the GIL, and
+// another thread's call then looks through the same vector: it must find it
+// whole, so the tensors are freed after they have left it.
+void forget(Call* c) {
+    std::vector<Call::Space> old;
+    old.swap(*c->spaces);
+}
+
 // The workspace kept for `stream`: the Python object's (ws_maker), remembered
 // here until it is told to forget.
 void* workspace_for(Call* c, void* stream, at::Tensor& hold) {
@@ -152,7 +160,7 @@ void* workspace_for(Call* c, void* stream, at::Tensor& hold) {
     }
     hold = THPVariable_Unpack(t);
     Py_DECREF(t);
-    if (c->spaces->size() >= 16) c->spaces->clear();
+    if (c->spaces->size() >= 16) forget(c);
     c->spaces->push_back({stream, hold});
     return hold.data_ptr();
 }
@@ -315,7 +323,7 @@ int call_clear(PyObject* self) {
     return 0;
 }
 PyObject* call_forget(PyObject* self, PyObject*) {
-    ((Call*)self)->spaces->clear();
+    forget((Call*)self);
     Py_RETURN_NONE;
 }
 PyMethodDef call_methods[] = {
