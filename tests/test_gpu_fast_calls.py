@@ -7,6 +7,7 @@ general path: same results, same conversions, same errors.
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import pytest
 import torch
@@ -151,3 +152,108 @@ def test_a_failed_launch_is_raised_and_not_made_again(entry, cuda_device, monkey
     assert calls == [entry]
     torch.cuda.synchronize()
     assert int(zeros.sum()) == 0
+
+
+@pytest.mark.parametrize("kv_dtype,precision,splits", [("fp8_e4m3fn", "auto", "auto"), ("fp8_e4m3fn", "fp8", 1),
+                                                       ("fp8_e4m3fn", "bf16", 3), ("bfloat16", "auto", "auto")])
+def test_history_call_takes_the_common_form_only(kv_dtype, precision, splits, cuda_device):
+    """The native call itself: it handles the common form (the general path
+    would hide that it does not) and gives up every other one."""
+    cfg, q, pool, table, valid, k_scale, v_scale = _case(cuda_device, kv_dtype)
+    kernel = make_history_attention_kernel(cfg)
+    want = kernel(q, pool, table, page_valid_len=valid.long(), k_scale=k_scale, v_scale=v_scale, precision=precision,
+                  splits=splits)
+    kernel(q, pool, table, page_valid_len=valid, k_scale=k_scale, v_scale=v_scale, precision=precision, splits=splits)
+    call = kernel._plans[precision, "fast", splits]
+    common = [q, pool, table, valid, k_scale, v_scale, None, False]
+
+    def run(**changed):
+        return call(*[changed.get(name, x) for name, x in zip(
+            ("q", "pool", "table", "valid", "k_scale", "v_scale", "out", "lse"), common)])
+
+    buffer = torch.empty_like(q)
+    for kw in ({}, {"table": table.long()}, {"out": buffer}, {"q": q.clone().requires_grad_()},
+               {"q": torch.nn.Parameter(q)}):
+        out = run(**kw)
+        assert type(out) is torch.Tensor and not out.requires_grad and torch.equal(out, want), kw
+    assert run(out=buffer) is buffer
+    out, lse = run(lse=True)
+    assert torch.equal(out, want) and lse.shape == q.shape[:3] and lse.dtype == torch.float32
+
+    class Subclass(torch.Tensor):
+        pass
+
+    for kw in ({"q": q.float()}, {"q": q.cpu()}, {"q": q.transpose(2, 3)}, {"q": q[:1]}, {"q": [q]},
+               {"q": q.as_subclass(Subclass)}, {"pool": pool.view(torch.uint8)}, {"pool": pool[:, :-1]},
+               {"table": table.cpu()}, {"table": table.float()}, {"table": table[:, :-1]}, {"valid": valid.long()},
+               {"valid": valid.cpu()}, {"k_scale": 1}, {"v_scale": torch.tensor(v_scale)}, {"out": q.float()},
+               {"out": q.cpu()}, {"lse": 1}):
+        assert run(**kw) is None, kw
+    seen = []
+    torch.vmap(lambda x: (seen.append(run(q=x)), x)[1])(q[None])  # a batched tensor has no storage
+    assert seen == [None]
+
+
+def test_other_calls_take_the_common_form_only(cuda_device):
+    cfg, q, pool, table, valid, _, _ = _case(cuda_device)
+    kv = torch.randn((2, 2, 128, 64), device=cuda_device, dtype=torch.bfloat16)
+    step = CurrentAttentionKernel(cfg)
+    out, lse = step(q, kv, return_lse=True)
+    assert torch.equal(step._fast(q, kv, None, None, None, False), out)
+    merged, _ = step._fast(q, kv, out, lse, out.clone(), True)
+    assert torch.equal(merged, step(q, kv, out, lse))
+    for args in ((q.float(), kv, None, None, None, False), (q, kv[:1], None, None, None, False),
+                 (q, kv, out, None, None, False), (q, kv, out, lse.double(), None, False),
+                 (q, kv, None, None, out.cpu(), False), (q, kv, None, None, None, 1)):
+        assert step._fast(*args) is None
+
+    x = torch.randn((2, 300, 64), device=cuda_device, dtype=torch.bfloat16)
+    writer = KVCacheWriter(cfg)
+    writer(x, x, pool, table, page_valid_len=valid)
+    common = (x, x, pool, table, 0, 1.0, 1.0, valid)
+    assert writer._fast(*common) == 0 and writer._fast(*common[:-1], None) == 0
+    assert writer._fast(x, x, pool, table.long(), *common[4:]) == 0
+    for at, other in ((0, x.float()), (0, x[0]), (1, x[:, :5].contiguous()), (2, pool.view(torch.uint8)),
+                      (3, table.cpu()), (4, -1), (4, 0.0), (4, 2**63), (5, 1), (6, torch.tensor(1.0)),
+                      (7, valid.long())):
+        assert writer._fast(*common[:at], other, *common[at + 1:]) is None, (at, other)
+
+    allocator = PageAllocator(cfg, cuda_device)
+    fresh = allocator.empty_table()
+    allocator.allocate(0, 10, fresh)
+    assert allocator._fast(0, 10, fresh, allocator.free_pages, allocator.free_count) == 0
+    assert allocator._fast(0, 10, fresh.long(), allocator.free_pages, allocator.free_count) == 0
+    for args in ((0, -1, fresh), (0.0, 10, fresh), (0, 2**31, fresh), (0, 10, fresh.cpu()), (0, 10, fresh[:, :1])):
+        assert allocator._fast(*args, allocator.free_pages, allocator.free_count) is None, args
+
+
+def test_threads_share_a_kernel_object(cuda_device):
+    """Calls of several threads on streams of their own, native and general,
+    with workspaces made and dropped meanwhile."""
+    cfg, q, pool, table, valid, k_scale, v_scale = _case(cuda_device)
+    kernel = make_history_attention_kernel(cfg)
+    options = [dict(precision=p, splits=s) for p in ("auto", "fp8", "bf16") for s in (1, 2, 3)]
+    kw = dict(k_scale=k_scale, v_scale=v_scale)
+    want = [make_history_attention_kernel(cfg)(q, pool, table, page_valid_len=valid.long(), **kw, **o) for o in options]
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(offset):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                got = []
+                for i in range(6 * len(options)):
+                    o = (offset + i) % len(options)
+                    lens = valid.long() if (offset + i) % 4 == 3 else valid
+                    got.append((o, kernel(q, pool, table, page_valid_len=lens, **kw, **options[o])))
+                torch.cuda.current_stream().synchronize()
+                assert all(torch.equal(out, want[o]) for o, out in got)
+        except BaseException as error:  # (raised in the test's own thread below)
+            errors.append(error)
+
+    threads = [threading.Thread(target=work, args=(3 * t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors

@@ -3,7 +3,8 @@
 Launches of few rows run workgroups of 128 rows and four waves, larger ones
 256 rows and eight waves.  A row's arithmetic does not depend on the shape, so
 the same rows must come out bit for bit from a small and from a large launch;
-both end inside row tiles and key tiles.
+both end inside row tiles and key tiles.  (head_dim 256; at 64 and 128 the tile
+kernel has one shape, and the launches differ in the tiles that a row shares.)
 """
 
 from __future__ import annotations
