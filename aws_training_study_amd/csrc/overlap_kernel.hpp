@@ -96,7 +96,7 @@ constexpr int threads(int waves) { return waves * 64; }
 
 template <int D>
 struct Shape {
-    static_assert(D == 128 || D == 256, "head_dim 128 or 256");
+    static_assert(D == 256, "head_dim 256");
     static constexpr int ROW = D;            // e4m3 bytes of one key row
     static constexpr int CHUNKS = D / 16;
     static constexpr int TILE = kKeyTile * ROW;
@@ -106,9 +106,8 @@ struct Shape {
     static constexpr int DT = D / 32;        // PV MFMAs per tile
     // Softmax micro-slices [pv_begin(i), pv_begin(i+1)) run beside PV MFMA i.
     static constexpr int pv_begin(int i) {
-        constexpr int b256[] = {0, 4, 6, 7, 8, 9, 10, 11, 14};
-        constexpr int b128[] = {0, 5, 8, 11, 14};
-        return D == 256 ? b256[i] : b128[i];
+        constexpr int begin[] = {0, 4, 6, 7, 8, 9, 10, 11, 14};
+        return begin[i];
     }
 };
 
@@ -798,18 +797,18 @@ __global__ void __launch_bounds__(threads(8), 1) history_fwd_overlap(FwdArgs a) 
     overlap_body<D, FAST, LSE, SPLIT, 8>(a, lds);
 }
 
-// Four waves, 128 rows.  The LDS (lds_bytes(D)) is dynamic so that the
+// Four waves, 128 rows.  The LDS (kDynamicLds) is dynamic so that the
 // compiler does not see that it leaves a CU one workgroup: it then keeps to
 // 256 VGPRs a wave.  With the four waves of a static 128 KB workgroup it took
 // 368 registers, the accumulators in AGPRs, and copied the scores out of them
 // (head_dim 256, 64 row tiles x 2 ranges of 16 key tiles: 46.4 us against 34;
 // workgroups of 256 rows 44.6).
-template <int D, bool FAST, bool LSE, bool SPLIT, int WAVES = 4>
-__global__ void __launch_bounds__(threads(WAVES), 8 / WAVES) history_fwd_overlap_waves(FwdArgs a) {
+template <int D, bool FAST, bool LSE, bool SPLIT>
+__global__ void __launch_bounds__(threads(4), 2) history_fwd_overlap_waves(FwdArgs a) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t dynamic_lds[];
-    overlap_body<D, FAST, LSE, SPLIT, WAVES>(a, dynamic_lds);
+    overlap_body<D, FAST, LSE, SPLIT, 4>(a, dynamic_lds);
 }
-constexpr int lds_bytes(int d) { return 2 * kStages * kKeyTile * d; }
+constexpr int kDynamicLds = 2 * Shape<256>::RING;
 
 }  // namespace ovl
 

@@ -308,7 +308,7 @@ inline int32_t history_launch(const pcpa_params* p, int splits, const void* q, c
     void* args[] = {&a};
     const int items = a.row_tiles * p->num_kv_heads * splits;
     const int threads = overlap ? ovl::threads(waves) : tile_threads(p->head_dim, fp8);
-    const size_t lds = narrow ? ovl::lds_bytes(p->head_dim) : 0;
+    const size_t lds = narrow ? ovl::kDynamicLds : 0;
     if (hipLaunchKernel(fn, dim3(8 * ((items + 7) / 8)), dim3(threads), args, lds, stream) != hipSuccess)
         return PCPA_ERR_LAUNCH;
     GuardShape g{};

@@ -445,9 +445,11 @@ class HistoryAttentionKernel:
             block_table = block_table.to(device=q.device, dtype=torch.int32).contiguous()
         return GraphedLaunch(lambda: self(q, kv_pages, block_table, block_valid_mask, **kwargs), warmup=warmup)
 
-    # Query rows per workgroup and workgroups per CU: the e4m3 head_dim-256
-    # kernel takes 256 rows and a whole CU; the tile kernel 128 rows, two
-    # per CU (one for BF16 MFMAs at head_dim 256).
+    # Query rows per workgroup and workgroups per CU that the split counts are
+    # chosen for: the e4m3 head_dim-256 kernel's 256 rows, a whole CU (a
+    # launch whose workgroups of 128 rows find a CU each takes those instead,
+    # after the splits are chosen); the tile kernel's 128 rows, two per CU
+    # (one for BF16 MFMAs at head_dim 256).
     ROWS_PER_WORKGROUP = {"overlap": 256, "tile": 128}
     # A split should still walk at least this many 64-key tiles (measured on
     # the MI355X: the overlap kernel's deeper pipeline needs longer ranges).
