@@ -14,7 +14,7 @@ namespace pcpa {
 // conversions (one per two elements) issue under the wave's own MFMAs.
 // Widening while staging instead, through registers, could not use the
 // LDS-DMA, nor overlap the next tile's loads: 16 ranks x 1024 tokens over 8192
-// keys at head_dim 256 took 309 us a call that way and take 229 (64% of the
+// keys at head_dim 256 took 308 us a call that way and take 230 (64% of the
 // bf16 MFMA peak at the clock held; the softmax finds few MFMAs of the other
 // wave on its SIMD to run under).  Two e4m3 terms for Q and P instead of
 // widened K and V are as fast but sum less exactly: the e4m3 MFMA's products
