@@ -158,7 +158,8 @@ void* workspace_for(Call* c, void* stream, at::Tensor& hold) {
         }
     PyObject* t = PyObject_CallFunction(c->ws_maker, "Ln", (long long)c->ws_bytes, (Py_ssize_t)(intptr_t)stream);
     if (!t) {
-        PyErr_Clear();
+        // an interrupt is the caller's; errors are the general path's to meet
+        if (PyErr_ExceptionMatches(PyExc_Exception)) PyErr_Clear();
         return nullptr;
     }
     hold = THPVariable_Unpack(t);
@@ -198,7 +199,10 @@ PyObject* history(Call* c, PyObject* const* a) {
     int32_t status;
     if (c->workspace) {
         void* const w = workspace_for(c, stream, ws);
-        if (!w) GIVE_UP;
+        if (!w) {
+            if (PyErr_Occurred()) return nullptr;
+            GIVE_UP;
+        }
         status = launch([&] {
             return ((HistorySplit)c->fn)(&p, c->n_split, qp, kp, tp, vp, op, lse_ptr, w, c->ws_bytes, stream);
         });

@@ -257,3 +257,25 @@ def test_threads_share_a_kernel_object(cuda_device):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+def test_an_interrupt_while_a_workspace_is_made_is_raised(cuda_device, monkeypatch):
+    """Errors of the workspace's maker leave the call to the general path, an
+    interrupt does not: it comes once."""
+    cfg, q, pool, table, valid, k_scale, v_scale = _case(cuda_device)
+    kernel = make_history_attention_kernel(cfg)
+    kw = dict(page_valid_len=valid, k_scale=k_scale, v_scale=v_scale)
+    make, raised = kernel._workspace, []
+
+    def once(*args, error):
+        if not raised:
+            raised.append(error)
+            raise error
+        return make(*args)
+
+    monkeypatch.setattr(kernel, "_workspace", lambda *args: once(*args, error=KeyboardInterrupt()))
+    with pytest.raises(KeyboardInterrupt):
+        kernel(q, pool, table, **kw)
+    raised.clear()
+    monkeypatch.setattr(kernel, "_workspace", lambda *args: once(*args, error=RuntimeError()))
+    assert kernel(q, pool, table, **kw).shape == q.shape and raised
